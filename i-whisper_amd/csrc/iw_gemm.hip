@@ -222,10 +222,13 @@ int gemm_dense(const GemmArgs &g, hipStream_t s) {
   const bool afast = g.K % 16 == 0 && g.lda % 16 == 0 && aligned16(g.a);
   const bool bfast = g.K % 16 == 0 && g.ldb % 16 == 0 && aligned16(g.b);
   if (gemm_skinny_eligible(g)) return gemm_skinny(g, nullptr, s);
+  // Above the decode kernels' rows the direct-to-LDS tiles, except for two
+  // chunks of rows over a long K (K = 5120, N = 1280: 12.7 / 13.9 us in chunks
+  // at 130 / 256 rows, 14.6 / 14.8 us in tiles; at K = 3072 the tiles win).
+  if (gemm_dtl_eligible(g) && !(g.M <= 2 * kSkinnyMaxRows && g.K >= 4096)) return gemm_dtl(g, s);
   if (g.M > kSkinnyMaxRows && g.M <= kSkinnyChunkMaxRows) {
-    // a few hundred rows (the decoder's prompt step): the decode kernel over
-    // chunks of 128 rows, whose launches cost less than one launch of the
-    // tile kernel at this size
+    // a few hundred rows: the decode kernel over chunks of 128 rows, whose
+    // launches cost less than one launch of the tile kernel at this size
     GemmArgs c = g;
     c.M = kSkinnyMaxRows;
     if (gemm_skinny_eligible(c)) {
@@ -241,7 +244,6 @@ int gemm_dense(const GemmArgs &g, hipStream_t s) {
       return 0;
     }
   }
-  if (g.M >= kBigGemmMinRows && gemm_dtl_eligible(g)) return gemm_dtl(g, s);
   if (afast && bfast && g.M >= kBigGemmMinRows) return gemm_big(g, false, s);
   switch (g.epi) {
     case EPI_L8:

@@ -209,7 +209,8 @@ constexpr int64_t kBigGemmMinRows = 8192;
 
 int gemm_dense(const GemmArgs &g, hipStream_t s);
 int gemm_big(const GemmArgs &g, bool conv_cl, hipStream_t s);
-// Direct-to-LDS kernel (iw_gemm_dtl.hip): dense A, K % 64 == 0, 16-byte aligned.
+// Direct-to-LDS kernels (iw_gemm_dtl.hip): dense A, K % 128 == 0 (64 from
+// kBigGemmMinRows rows), N % 16 == 0, 16-byte aligned.
 bool gemm_dtl_eligible(const GemmArgs &g);
 int gemm_dtl(const GemmArgs &g, hipStream_t s);
 int gemm_conv(const GemmArgs &g, bool channels_last, hipStream_t s);

@@ -1,0 +1,10 @@
+// The direct-to-LDS GEMM (iw_gemm_dtl.hpp) on 64 x 128 tiles.
+#include "iw_gemm_dtl.hpp"
+
+namespace iw {
+namespace dtl {
+
+template int gemm_dtl_tile<Tile64x128>(const GemmArgs &, hipStream_t);
+
+}  // namespace dtl
+}  // namespace iw

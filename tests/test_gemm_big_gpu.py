@@ -212,3 +212,45 @@ def test_linear8_dtl_edge_shapes(iw, oracle, gpu, M, K, N, kind):
         exp = oracle.linear8(x, w, b, z, m, s)
     assert np.array_equal(host(got), exp)
     assert len(np.unique(exp)) > (20 if kind == "gelu_table" else 50)
+
+
+# The smaller direct-to-LDS tiles (K % 128 == 0, more than 128 rows): one row
+# past the decode kernels, edges of 64- and 128-row and -column tiles, one,
+# two, an odd number of and many 128-byte stages, every epilogue.
+@pytest.mark.parametrize("M,K,N", [(129, 128, 16), (257, 256, 80), (449, 384, 1152), (1500, 640, 1296),
+                                   (2047, 1280, 400), (3001, 384, 2064), (300, 4096, 144), (700, 5120, 1280)])
+@pytest.mark.parametrize("kind", ["l8", "l8_sym", "gelu_table", "gelu", "l32", "l32res", "classifier"])
+def test_gemm_dtl_small_tiles(iw, oracle, gpu, kind, M, K, N):
+    print("case: gemm dtl small tiles", kind, M, K, N, flush=True)
+    seed = 7 * M + 11 * K + N + len(kind)
+    x, w, b, z, m, s = gen.realistic_linear_case(seed, M, K, N, asym=kind != "l8_sym")
+    if kind in ("l8", "l8_sym"):
+        s[:4] = [-2, 0, 33, 31]
+        m[5] = 0xC0000001  # its tile takes the high-product correction
+        got = iw.kernels.linear8_hip(T(x), T(w), T(b), None if z is None else T(z), T(m), T(s))
+        exp = oracle.linear8(x, w, b, z, m, s)
+    elif kind in ("gelu_table", "gelu"):
+        n = N if kind == "gelu" else 1  # per channel, or one value (the table form)
+        lut = np.round(255 / (1 + np.exp(-np.arange(-6, 6, 0.75)))).astype(np.uint8)
+        im, om = (v + np.arange(n) % 5 for v in (93, 64))
+        im, om, is_, os_ = im.astype(np.uint8), om.astype(np.uint8), np.full(n, 10, np.int8), np.full(n, 14, np.int8)
+        got = iw.kernels.linear8_gelu_hip(T(x), T(w), T(b), T(z), T(m), T(s), T(lut), T(im), T(is_), T(om), T(os_))
+        exp = oracle.gelu(oracle.linear8(x, w, b, z, m, s), lut, im, is_, om, os_)
+    elif kind == "l32":
+        got = iw.kernels.linear32_hip(T(x), T(w), T(b), T(z), T(m), T(s))
+        exp = oracle.linear32(x, w, b, z, m, s)
+    elif kind == "classifier":
+        got = iw.kernels.classifier_hip(T(x)[None], T(w), torch.tensor([int(m[0])], dtype=torch.uint32),
+                                        torch.tensor([int(s[6])], dtype=torch.int8))[0]
+        exp = oracle.classifier(x, w, int(m[0]), int(s[6]))
+    else:
+        s[:] = np.arange(N) % 4
+        r = gen.rng(seed + 1)
+        res = r.integers(-16383, 16384, size=(M, N)).astype(np.int16)
+        rm = int(r.integers(1, 65536))
+        exp = oracle.residual15(oracle.linear32(x, w, b, z, m, s), res, rm)
+        got = T(res)
+        iw.kernels.linear32_residual15_hip(T(x), T(w), T(b), T(z), T(m), T(s), got,
+                                           torch.tensor([rm], dtype=torch.uint16), out=got)
+    assert np.array_equal(host(got), exp)
+    assert len(np.unique(exp)) > 20
