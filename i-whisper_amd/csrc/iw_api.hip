@@ -622,13 +622,14 @@ int iw_attention(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, i
   IW_REQUIRE(table, "prefill attention needs the shift-exp table");
   IW_REQUIRE(v_sh == head_dim * v_sd && v_sb == heads * head_dim * v_sd,
              "prefill attention expects V^T as [B,H,D,v_sd]");
+  if (attn_prefill_split_eligible(a)) return launch_attn_prefill_split(a, as_stream(stream));
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) {
     int v = 0;
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
       cus = v;
   }
-  return launch_attn_prefill(a, cus * (head_dim <= 64 ? 4 : 3), as_stream(stream));
+  return launch_attn_prefill(a, cus * 4, as_stream(stream));
 }
 
 int iw_transpose_heads(const int8_t *src, int64_t src_sb, int64_t src_st, int8_t *dst,

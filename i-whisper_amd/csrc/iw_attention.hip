@@ -15,6 +15,7 @@
 //                   tensors are never written to memory.
 //   attn_decode   - streaming kernel for a few query rows over a KV cache
 //                   (decoder self- and cross-attention).
+#include "iw_attn_dev.hpp"
 #include "iw_common.hpp"
 #include "iw_gemm.hpp"
 #include "iw_kernels.hpp"
@@ -30,11 +31,6 @@ namespace {
 // out-projection GEMM.
 __device__ __forceinline__ int64_t decode_out_index(const AttnArgs &a, int64_t b, int c) {
   return a.o_frag_kp ? frag_offset(b, c, a.o_frag_kp) : b * a.o_sb + c;
-}
-
-__device__ __forceinline__ int32_t qk_requant16(int32_t acc, uint32_t m, uint32_t s) {
-  // (int32)(acc * m) modulo 2^32, Rshift, saturate to int16
-  return clampi(rshift((int32_t)((uint32_t)acc * m), s), -32768, 32767);
 }
 
 // ------------------------------------------------------------------------
@@ -147,14 +143,6 @@ __global__ void shift_exp_lut_kernel(uint8_t *lut, int32_t f) {
 
 constexpr int PF_KC = 64;  // keys per LDS stage
 
-// Median of three signed ints: clamp of x to [lo, hi] for lo <= hi, in one
-// instruction where the bounds are not compile-time constants.
-__device__ __forceinline__ int32_t med3i(int32_t x, int32_t lo, int32_t hi) {
-  int32_t r;
-  asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(lo), "v"(hi));
-  return r;
-}
-
 __device__ __forceinline__ int key_row(int kk) {
   // LDS row of key kk (0..31) inside a 32-key sub-block
   const int g = kk >> 4, r = kk & 15;
@@ -164,7 +152,7 @@ __device__ __forceinline__ int key_row(int kk) {
 // DF: the head dim is exactly 32 KS, so whole-chunk K / V^T copies need no
 // bounds tests.
 template <int KS, bool HAS_MASK, bool DF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KS <= 2 ? 4 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void attn_prefill_kernel(AttnArgs a) {
   constexpr int DP = KS * 32;           // padded head dim
   // K and V^T rows of 4 chunks of 16 bytes (head_dim 64) are unpadded, with
@@ -349,32 +337,10 @@ void attn_prefill_kernel(AttnArgs a) {
     for (; kc1 < nkc; ++kc1) pass1(kc1, No{}, No{});
     mx = max(mx, __shfl_xor(mx, 32));
     const int32_t rowmax = mx == INT32_MIN ? -32768 : qk_requant16(mx, a.qk_m, a.qk_s);
-    const uint32_t rmp1 = (uint32_t)(uint16_t)(rowmax + 1);
 
-    // ---- pass 2: P = E(S - rmp1) and O = P . V ----
-    // requant constants (a shift >= 32 gives 0: multiplier 0 instead)
-    const int32_t qm24 = a.qk_s >= 32 ? 0 : (int32_t)a.qk_m;
-    const uint32_t qsh = a.qk_s >= 32 ? 0u : a.qk_s;
-    const uint32_t qhalf = qsh ? 1u << (qsh - 1) : 0u;
-    const uint32_t qw = min(qsh, 1u);
-    // Keys of a full chunk all count in the row maximum, so with the row
-    // maximum below 32767 rowmax + 1 - h16 lies in [1, 65535] and the table
-    // index is
-    //   min(R - clamp16(h), L) = med3(R - h, min(R - 32767, L), min(R + 32768, L))
-    // with R = rowmax + 1 and h the unsaturated shift. R - h itself is one
-    // shift: with v = s * m, h = (v + half - [v < 0]) >> sh (floor), and
-    //   R - h = (R * 2^sh + 2^sh - 1 - half - v + [v < 0]) >> sh   (floor),
-    // which stays inside int32: |v| <= 2^21 * 255 < 2^29 and |R| <= 2^(29 - sh) + 2
-    // for sh <= 29. For sh >= 30 every h is 0 (|v| < 2^29 <= half), the same
-    // as m = 0 with sh = 0. [v < 0] = [s < 0] when m > 0; when m = 0 the term
-    // is below the rounding step either way (2^sh - half <= 2^sh - 1).
-    const uint32_t fsh = a.qk_s >= 30 ? 0u : a.qk_s;
-    const int32_t fnm = a.qk_s >= 30 ? 0 : -(int32_t)a.qk_m;
-    const uint32_t fw = min(fsh, 1u);
-    const int32_t fR = rowmax + 1;
+    // ---- pass 2: P = E(S - rowmax - 1) and O = P . V ----
+    const ScoreIndex ix(a, rowmax);
     const bool no_sat = !__any(rowmax >= 32767);
-    const int32_t fK = (int32_t)(((uint32_t)fR << fsh) + ((1u << fsh) - 1u) - (fsh ? 1u << (fsh - 1) : 0u));
-    const int32_t flo = min(fR - 32767, IW_SEXP_LUT - 1), fhi = min(fR + 32768, IW_SEXP_LUT - 1);
     v16i o[KS];
 #pragma unroll
     for (int t = 0; t < KS; ++t)
@@ -405,26 +371,12 @@ void attn_prefill_kernel(AttnArgs a) {
       for (int sub = 0; sub < 2; ++sub) {
         const v16i s = scores(sub);
         const int kbase0 = kc * PF_KC + sub * 32 + g * 16;
-        // P of the 16 keys: requant (24-bit product: |score| < 2^21 and an
-        // 8-bit multiplier), round-half-away shift, int16 saturation, then
-        // the table at min((rowmax + 1 - h16) mod 2^16, size - 1)
-        // (keys past Tk or masked: P = 0, applied as a byte mask on the
-        // loaded value rather than a conditional write)
+        // P of the 16 keys (keys past Tk or masked: P = 0, applied as a byte
+        // mask on the loaded value rather than a conditional write)
         uint32_t pb[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          uint32_t idx;
-          if constexpr (FULL) {
-            const uint32_t y = (uint32_t)(__mul24(s[r], fnm) + fK) -
-                               (uint32_t)__builtin_amdgcn_sbfe(s[r], 31, fw);
-            idx = (uint32_t)med3i((int32_t)y >> fsh, flo, fhi);
-          } else {
-            const int32_t v = __mul24(s[r], qm24);
-            const uint32_t tr = (uint32_t)v + qhalf + (uint32_t)__builtin_amdgcn_sbfe(v, 31, qw);
-            const int32_t h16 = clampi((int32_t)tr >> qsh, -32768, 32767);
-            idx = min((rmp1 - (uint32_t)h16) & 0xffffu, (uint32_t)(IW_SEXP_LUT - 1));
-          }
-          pb[r] = (uint32_t)sLut[idx];
+          pb[r] = (uint32_t)sLut[FULL ? ix.full(s[r]) : ix.any(s[r])];
           if constexpr (!FULL) {
             const int key = kbase0 + r;
             bool ok = key < a.Tk;
@@ -1570,9 +1522,7 @@ int launch_attn_prefill(const AttnArgs &a, int max_blocks, hipStream_t s) {
   switch (ks) {
     case 1: IW_PF(1) break;
     case 2: IW_PF(2) break;
-    case 3: IW_PF(3) break;
-    case 4: IW_PF(4) break;
-    default: return fail("fused attention supports head_dim <= 128");
+    default: return fail("this prefill kernel takes head_dim <= 64");
   }
 #undef IW_PF
   return check_launch("attn_prefill_kernel");

@@ -137,6 +137,10 @@ int launch_pv_norm_requant(const uint8_t *p, const int8_t *v, const int32_t *row
                            int64_t tq, int64_t tk, int64_t dim, hipStream_t s);
 int launch_shift_exp_lut(uint8_t *lut, int32_t f, hipStream_t s);
 int launch_attn_prefill(const AttnArgs &a, int max_blocks, hipStream_t s);
+// the same with the keys of 32-query tiles split over a block's waves, and
+// where that is the faster form (iw_attn_split.hip)
+bool attn_prefill_split_eligible(const AttnArgs &a);
+int launch_attn_prefill_split(const AttnArgs &a, hipStream_t s);
 int launch_attn_decode(const AttnArgs &a, hipStream_t s);
 // Decode attention over [B,H,T_cap,D] / [B,H,D,T_cap16] caches; key count
 // a.Tk + *pos (pos may be null). At most 4096 keys.

@@ -445,6 +445,29 @@ def test_attention_prefill_wrap_in_full_chunks(iw, oracle, gpu):
         assert np.array_equal(got, exp), qs
 
 
+# The prefill kernel by number of 32-query tiles: keys split over a block's
+# waves (one or two tiles a wave), or 128 queries per block; with ragged and
+# full key chunks, saturated row maxima (P = 128) beside ordinary rows, head
+# dims that fill an MFMA step or not, and fully masked query rows.
+@pytest.mark.parametrize("B,H", [(1, 3), (10, 28), (20, 28)])
+@pytest.mark.parametrize("Tq,Tk,D", [(65, 150, 64), (70, 64, 64), (96, 97, 32), (65, 33, 48), (67, 130, 96),
+                                     (65, 40, 128), (32, 290, 64), (1, 31, 80)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_prefill_tile_counts(iw, oracle, gpu, B, H, Tq, Tk, D, masked):
+    _print_case("attention prefill tiles", B, H, Tq, Tk, D, masked)
+    q, k, v, qm, qs, f, am, as_ = gen.attn_case(11 * B + Tq + 3 * Tk + D, B, H, Tq, Tk, D)
+    q[0, :, : Tq // 2] = 127  # these rows' scores reach the int16 maximum at shift 0 of the second pass
+    k[0, :, ::3] = 127
+    mask = None
+    if masked:
+        mask = gen.rng(Tq).random((Tq, Tk)) < 0.3
+        mask[Tq // 3] = True
+    for shift in (qs, 0):
+        exp = oracle.attention(q, k, v, mask, qm, shift, f, am, as_)
+        got = _fused(iw, q, k, v, mask, qm, shift, f, am, as_, decode=False)
+        assert np.array_equal(got, exp), shift
+
+
 def test_argmax_rows(iw, gpu):
     r = gen.rng(9)
     x = gen.i8(r, (7, 51865))
