@@ -584,28 +584,35 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 // K cache [B, H, T_cap, D] (rows of D bytes contiguous per head), V cache
 // transposed [B, H, D, T_cap16]. The key count is k_length, plus *pos when
 // pos is given (the self-attention cache length lives on the device, so a
-// captured decode step can be replayed). One block of 256 threads per
+// captured decode step can be replayed). One block of NWV waves per
 // (batch, head):
 //   1. scores: LPK lanes share a key (16 bytes each), so one wave load reads
 //      64 / LPK consecutive keys; raw int32 scores go to LDS and their max
 //      gives the row max (the requant is monotone);
 //   2. P = shift_exp(requant(s) - row_max - 1) to LDS, with its row sum;
-//   3. O[d] = sum_j P[j] V^T[d][j]: each wave owns D / 4 rows of V^T and its
+//   3. O[d] = sum_j P[j] V^T[d][j]: each wave owns D / NWV rows of V^T and its
 //      lanes walk a row's 16-byte chunks, so each wave load reads 1 KB of one
 //      row; the per-lane partial sums are reduced once per row.
 constexpr int DC_MAX_TK = 4096;
+// Up to one block per CU 16 waves share a (batch, head), with every key load of
+// a 1500-key cache in flight; else 4. Head dim 96, us: 4 blocks 20.2 -> 13.4, 256
+// blocks 28.8 -> 25.1.
+constexpr int64_t kManyWavesBlocks = 256;
 
-template <int D, int PRE>
-__global__ __launch_bounds__(256) void attn_decode_cache_kernel(AttnArgs a, const int32_t *pos) {
+// NWV: waves per (batch, head).
+template <int D, int PRE, int NWV>
+__global__ __launch_bounds__(64 * NWV) void attn_decode_cache_kernel(AttnArgs a, const int32_t *pos) {
   constexpr int CPK = D / 16;                      // 16-byte chunks per key
   constexpr int LPK = CPK <= 4 ? 4 : 8;            // lanes per key
   constexpr int KPW = 64 / LPK;                    // keys per wave load
-  constexpr int RPW = D / 4;                       // V^T rows per wave
-  constexpr int UK = 4;                            // key loads in flight per lane
+  constexpr int RPW = D / NWV;                     // V^T rows per wave
+  constexpr int UK = NWV == 4 ? 4 : 12;            // key loads in flight per lane
+  constexpr int NT = 64 * NWV;
+  static_assert(D % NWV == 0, "whole V^T rows per wave");
   __shared__ int32_t sS[DC_MAX_TK];
   __shared__ __attribute__((aligned(16))) uint8_t sP[DC_MAX_TK];
-  __shared__ int32_t sRed[4];
-  __shared__ uint32_t sSum[4];
+  __shared__ int32_t sRed[NWV];
+  __shared__ uint32_t sSum[NWV];
   __shared__ uint32_t sHi;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -638,18 +645,18 @@ __global__ __launch_bounds__(256) void attn_decode_cache_kernel(AttnArgs a, cons
     qv = *reinterpret_cast<const v4i *>(a.q + b * a.q_sb + (int64_t)h * D + chunk * 16);
   const int8_t *kb = a.k + b * a.k_sb + (int64_t)h * a.k_sh;
   int32_t mx = INT32_MIN;
-  for (int j0 = wave * KPW; j0 < Tk; j0 += 4 * KPW * UK) {
+  for (int j0 = wave * KPW; j0 < Tk; j0 += NWV * KPW * UK) {
     v4i kv[UK];
 #pragma unroll
     for (int u = 0; u < UK; ++u) {
-      const int j = j0 + u * 4 * KPW + lane / LPK;
+      const int j = j0 + u * NWV * KPW + lane / LPK;
       kv[u] = (j < Tk && cvalid)
                   ? *reinterpret_cast<const v4i *>(kb + (int64_t)j * a.k_st + chunk * 16)
                   : v4i{0, 0, 0, 0};
     }
 #pragma unroll
     for (int u = 0; u < UK; ++u) {
-      const int j = j0 + u * 4 * KPW + lane / LPK;
+      const int j = j0 + u * NWV * KPW + lane / LPK;
       int32_t acc = 0;
       acc = __builtin_amdgcn_sdot4(qv[0], kv[u][0], acc, false);
       acc = __builtin_amdgcn_sdot4(qv[1], kv[u][1], acc, false);
@@ -667,13 +674,14 @@ __global__ __launch_bounds__(256) void attn_decode_cache_kernel(AttnArgs a, cons
   for (int off = 32; off >= 1; off >>= 1) mx = max(mx, __shfl_xor(mx, off));
   if (lane == 0) sRed[wave] = mx;
   __syncthreads();
-  mx = max(max(sRed[0], sRed[1]), max(sRed[2], sRed[3]));
+#pragma unroll
+  for (int w = 0; w < NWV; ++w) mx = max(mx, sRed[w]);
   const int32_t rowmax = mx == INT32_MIN ? -32768 : qk_requant16(mx, a.qk_m, a.qk_s);
   const uint32_t rmp1 = (uint32_t)(uint16_t)(rowmax + 1);
 
   // ---- phase 2: P and its row sum ----
   uint32_t psum = 0, hi = 0;
-  for (int j = tid; j < tk16; j += 256) {
+  for (int j = tid; j < tk16; j += NT) {
     uint32_t p = 0;
     if (j < Tk) {
       const int32_t h16 = qk_requant16(sS[j], a.qk_m, a.qk_s);
@@ -689,7 +697,10 @@ __global__ __launch_bounds__(256) void attn_decode_cache_kernel(AttnArgs a, cons
   if (lane == 0) sSum[wave] = psum;
   if (hi & 0x80u) atomicOr(&sHi, 1u);
   __syncthreads();
-  const int32_t total = (int32_t)(sSum[0] + sSum[1] + sSum[2] + sSum[3]);
+  uint32_t tot = 0;
+#pragma unroll
+  for (int w = 0; w < NWV; ++w) tot += sSum[w];
+  const int32_t total = (int32_t)tot;
   const int32_t inv = fisr(total, a.rsqrt_off);
   const bool any_hi = sHi != 0;
 
@@ -789,6 +800,17 @@ __global__ __launch_bounds__(256) void attn_decode_cache_kernel(AttnArgs a, cons
 #ifndef IW_DS_CH
 #define IW_DS_CH 128
 #endif
+// Grids of at most one block per CU take 16 waves per (batch, head), 256-key
+// chunks and four slots (64 KB): there a block has its CU to itself and what
+// bounds it is the chain of its own steps, four times shorter per wave (a
+// deeper ring for the four waves changes nothing). us per launch over 1500
+// HBM-cold keys: 20 blocks 11.0 -> 8.2, 256 blocks 14.4 -> 12.2; three queries
+// 24.6 -> 16.1; with LayerNorm and query 14.8 -> 11.8 and 17.3 -> 15.2. From two
+// blocks per CU the chains of several small blocks overlap and the forms
+// tie (324 blocks: 17.1 and 17.8).
+constexpr int DM_NW = 16, DM_NR = 4, DM_CH = 256;
+constexpr int64_t kManyWavesMaxBlocks = 256;
+
 // the self-attention instance (at most 512 keys) has its own ring shape
 #ifndef IW_DSS_NR
 #define IW_DSS_NR 3
@@ -816,44 +838,51 @@ constexpr int kSelfTailBlocks = 128;
 
 // The query of (batch b, head h) for attn_decode_cross_lnq_kernel, as 64
 // bytes of LDS: LayerNorm32 of row b (the integer steps of
-// layernorm32_row_kernel: thread t owns elements t, t + 256, ..., three
+// layernorm32_row_kernel: thread t of 64 NW owns elements t, t + 64 NW, ..., three
 // reduction rounds) into the LDS row hb, then Linear8 of the head's 64
-// channels: wave w takes the k32 steps s = w, w + 4, ... of both 32-channel
+// channels: wave w takes the k32 steps s = w, w + NW, ... of both 32-channel
 // fragment rows of wq (lane l: channel 32 r + l % 32, bytes 32 s + 16 (l / 32)
 // .. +15, against the same bytes of hb), the partial sums meet in LDS
 // (ds_add, modulo 2^32) and threads 0-63 apply the Linear8 epilogue with the
 // row sum of hb for the zero-point term. The row, the parameters and the
-// first five steps' weight fragments are requested first (ln_query_load),
+// first steps' weight fragments are requested first (ln_query_load),
 // ahead of the block's first K/V chunk copies, so that the LayerNorm waits
-// for its own loads only; the other five steps' fragments after it.
+// for its own loads only; the other steps' fragments after it.
+// NW waves: E row elements per thread; of a wave's k32 steps (at most 40 / NW)
+// H are in registers at once.
+template <int NW>
 struct LnqRegs {
-  int32_t v[5], gm[5], bt[5];
+  static constexpr int E = (1280 + 64 * NW - 1) / (64 * NW), STEPS = (40 + NW - 1) / NW, H = STEPS < 5 ? STEPS : 5;
+  static_assert(STEPS % H == 0, "whole groups of steps");
+  int32_t v[E], gm[E], bt[E];
   int32_t qb, qz, qs;
   uint32_t qm;
-  v4i f0[5], f1[5];
+  v4i f0[H], f1[H];
 };
 
-__device__ __forceinline__ void lnq_frags(const LnQueryArgs &lq, int h, int half, v4i (&f0)[5], v4i (&f1)[5]) {
+template <int NW>
+__device__ __forceinline__ void lnq_frags(const LnQueryArgs &lq, int h, int half, LnqRegs<NW> &r) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nst = (int)(lq.kp >> 5);  // k32 steps (the padding has zero weights)
   const int8_t *w0 = lq.wq + ((int64_t)(2 * h) * nst) * 1024 + lane * 16;
   const int8_t *w1 = w0 + (int64_t)nst * 1024;
 #pragma unroll
-  for (int t = 0; t < 5; ++t) {
-    const int st = wave + 4 * (5 * half + t);
+  for (int t = 0; t < LnqRegs<NW>::H; ++t) {
+    const int st = wave + NW * (LnqRegs<NW>::H * half + t);
     const int sc = st < nst ? st : 0;
-    f0[t] = *reinterpret_cast<const v4i *>(w0 + (int64_t)sc * 1024);
-    f1[t] = *reinterpret_cast<const v4i *>(w1 + (int64_t)sc * 1024);
+    r.f0[t] = *reinterpret_cast<const v4i *>(w0 + (int64_t)sc * 1024);
+    r.f1[t] = *reinterpret_cast<const v4i *>(w1 + (int64_t)sc * 1024);
   }
 }
 
-__device__ __forceinline__ void ln_query_load(const LnQueryArgs &lq, int64_t b, int h, LnqRegs &r) {
+template <int NW>
+__device__ __forceinline__ void ln_query_load(const LnQueryArgs &lq, int64_t b, int h, LnqRegs<NW> &r) {
   const int tid = threadIdx.x;
   const int C = lq.hidden;
   const int16_t *xr = lq.x + b * lq.ldx;
 #pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    const int e = tid + 256 * j;
+  for (int j = 0; j < LnqRegs<NW>::E; ++j) {
+    const int e = tid + 64 * NW * j;
     const bool ok = e < C;
     r.v[j] = ok ? xr[e] : 0;
     r.gm[j] = ok ? lq.gamma[e] : 0;
@@ -865,14 +894,14 @@ __device__ __forceinline__ void ln_query_load(const LnQueryArgs &lq, int64_t b, 
   r.qz = lq.wz ? (int32_t)lq.wz[n] : 0;
   r.qm = lq.mult[n];
   r.qs = lq.shift[n];
-  lnq_frags(lq, h, 0, r.f0, r.f1);
+  lnq_frags<NW>(lq, h, 0, r);
 }
 
 // The normalised row (up to 1280 bytes) and the query sums (64 words) use
 // sP, which the attention first writes after the scores.
-__device__ __forceinline__ const int8_t *ln_query(const LnQueryArgs &lq, LnqRegs &r, int h, uint8_t *sP) {
-  constexpr int NWV = 4;
-  __shared__ uint32_t sLn[3][NWV];  // the LayerNorm's wave partials
+template <int NW>
+__device__ __forceinline__ const int8_t *ln_query(const LnQueryArgs &lq, LnqRegs<NW> &r, int h, uint8_t *sP) {
+  __shared__ uint32_t sLn[3][NW];  // the LayerNorm's wave partials
   __shared__ __attribute__((aligned(16))) int8_t q8[64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int C = lq.hidden;
@@ -883,42 +912,49 @@ __device__ __forceinline__ const int8_t *ln_query(const LnQueryArgs &lq, LnqRegs
 
   uint32_t sum = 0;
 #pragma unroll
-  for (int j = 0; j < 5; ++j) sum += (uint32_t)r.v[j];
+  for (int j = 0; j < LnqRegs<NW>::E; ++j) sum += (uint32_t)r.v[j];
   sum = wave_sum_dpp(sum);
   if (lane == 0) sLn[0][wave] = sum;
   lds_barrier();
-  const int32_t mean = norm_reduce((int32_t)(sLn[0][0] + sLn[0][1] + sLn[0][2] + sLn[0][3]), lq.code);
+  auto total = [&](int i) {
+    uint32_t t = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t += sLn[i][w];
+    return (int32_t)t;
+  };
+  const int32_t mean = norm_reduce(total(0), lq.code);
   int32_t maxsq = 0;
 #pragma unroll
-  for (int j = 0; j < 5; ++j)
-    if (tid + 256 * j < C) {
+  for (int j = 0; j < LnqRegs<NW>::E; ++j)
+    if (tid + 64 * NW * j < C) {
       const int32_t d = r.v[j] - mean;
       maxsq = max(maxsq, (int32_t)((uint32_t)d * (uint32_t)d));
     }
   maxsq = wave_max_dpp(maxsq);
   if (lane == 0) sLn[1][wave] = (uint32_t)maxsq;
   lds_barrier();
-  maxsq = max(max((int32_t)sLn[1][0], (int32_t)sLn[1][1]), max((int32_t)sLn[1][2], (int32_t)sLn[1][3]));
+#pragma unroll
+  for (int w = 0; w < NW; ++w) maxsq = max(maxsq, (int32_t)sLn[1][w]);
   int32_t rs = bitlen(maxsq) - 16;
   rs = rs < 0 ? 0 : rs;
   rs = (rs + 1) & ~1;
   uint32_t vs = 0;
 #pragma unroll
-  for (int j = 0; j < 5; ++j)
-    if (tid + 256 * j < C) {
+  for (int j = 0; j < LnqRegs<NW>::E; ++j)
+    if (tid + 64 * NW * j < C) {
       const int32_t d = r.v[j] - mean;
       vs += (uint32_t)rshift((int32_t)((uint32_t)d * (uint32_t)d), (uint32_t)rs);
     }
   vs = wave_sum_dpp(vs);
   if (lane == 0) sLn[2][wave] = vs;
   lds_barrier();
-  const int32_t var = norm_reduce((int32_t)(sLn[2][0] + sLn[2][1] + sLn[2][2] + sLn[2][3]), lq.code);
+  const int32_t var = norm_reduce(total(2), lq.code);
   const int32_t inv = fisr(var, lq.rsqrt_off);
   const uint32_t nshift = (uint32_t)(lq.ln_s + (rs >> 1));
   uint32_t rsum = 0;
 #pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    const int e = tid + 256 * j;
+  for (int j = 0; j < LnqRegs<NW>::E; ++j) {
+    const int e = tid + 64 * NW * j;
     if (e < C) {
       const int32_t d = r.v[j] - mean;
       const uint32_t t = (uint32_t)d * (uint32_t)inv * lq.ln_m;
@@ -938,29 +974,32 @@ __device__ __forceinline__ const int8_t *ln_query(const LnQueryArgs &lq, LnqRegs
   const int nst = (int)(lq.kp >> 5);
   const int hoff = 16 * (lane >> 5);
   int32_t acc0 = 0, acc1 = 0;
-  auto dot = [&](int half, const v4i (&f0)[5], const v4i (&f1)[5]) {
+  auto dot = [&](int half) {
 #pragma unroll
-    for (int t = 0; t < 5; ++t) {
-      const int st = wave + NWV * (5 * half + t);
+    for (int t = 0; t < LnqRegs<NW>::H; ++t) {
+      const int st = wave + NW * (LnqRegs<NW>::H * half + t);
       if (st < nst) {
         const v4i hv = *reinterpret_cast<const v4i *>(hb + 32 * st + hoff);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          acc0 = __builtin_amdgcn_sdot4(f0[t][e], hv[e], acc0, false);
-          acc1 = __builtin_amdgcn_sdot4(f1[t][e], hv[e], acc1, false);
+          acc0 = __builtin_amdgcn_sdot4(r.f0[t][e], hv[e], acc0, false);
+          acc1 = __builtin_amdgcn_sdot4(r.f1[t][e], hv[e], acc1, false);
         }
       }
     }
   };
-  // then steps 5..9 of each wave (kp <= 1280: at most ten per wave)
-  dot(0, r.f0, r.f1);
-  lnq_frags(lq, h, 1, r.f0, r.f1);
-  dot(1, r.f0, r.f1);
+  // then each wave's further steps (kp <= 1280)
+  dot(0);
+#pragma unroll
+  for (int i = 1; i < LnqRegs<NW>::STEPS / LnqRegs<NW>::H; ++i) {
+    lnq_frags<NW>(lq, h, i, r);
+    dot(i);
+  }
   atomicAdd(&qacc[lane & 31], acc0);
   atomicAdd(&qacc[32 + (lane & 31)], acc1);
   lds_barrier();
   if (tid < 64) {
-    const int32_t xsum = (int32_t)(sLn[0][0] + sLn[0][1] + sLn[0][2] + sLn[0][3]);
+    const int32_t xsum = total(0);
     // acc - wz * rowsum + bias modulo 2^32 (|rowsum| <= 127 C < 2^23: exact
     // in the 24-bit multiplier), then the Linear8 requantization
     const uint32_t corr = (uint32_t)qacc[tid] - (uint32_t)__mul24(r.qz, xsum) + (uint32_t)r.qb;
@@ -984,7 +1023,7 @@ __device__ __forceinline__ void attn_decode_stream_body(const AttnArgs &a, const
   constexpr int NACC = VQ ? 4 : DPC;  // P.V sums per lane
   static_assert(!VQ || NW * 64 * 4 <= MAXK * 2, "the wave sums of P.V fit in the score array");
   static_assert(NQ == 1 || !VQ, "several queries stream V transposed");
-  static_assert(!LNQ || (NQ == 1 && !VQ && NW == 4), "the fused query: one, V transposed");
+  static_assert(!LNQ || (NQ == 1 && !VQ), "the fused query: one, V transposed");
   // the fused query's LayerNorm keeps its normalised row (up to 1280 bytes) and the 64 query
   // channels' int32 sums (at byte 1280) in sP
   static_assert(!LNQ || NQ * MAXK >= 1280 + 64 * (int)sizeof(int32_t), "the fused query's row and sums fit in sP");
@@ -1046,8 +1085,8 @@ __device__ __forceinline__ void attn_decode_stream_body(const AttnArgs &a, const
     for (int u = 0; u < DPC; ++u)
       dma16_lds(a.q + b * a.q_sb + (int64_t)h * D + cq * 16, ring + (NR - 1) * SLOT + u * 1024);
   }
-  LnqRegs lr;
-  if constexpr (LNQ) ln_query_load(lq, b, h, lr);
+  LnqRegs<NW> lr;
+  if constexpr (LNQ) ln_query_load<NW>(lq, b, h, lr);
   // LNQ: the last slot holds no copied query, so chunk NR - 1 is copied now
   // too, during the LayerNorm and projection (the loop then issues chunk
   // i + NR - 1 from i = 1 on; at i = 0 its wait also covers chunk 1)
@@ -1055,7 +1094,7 @@ __device__ __forceinline__ void attn_decode_stream_body(const AttnArgs &a, const
   for (int i = 0; i < (LNQ ? NR : NR - 1); ++i)
     if (i < T) issue(i);
   const int8_t *q8 = nullptr;
-  if constexpr (LNQ) q8 = ln_query(lq, lr, h, sP);
+  if constexpr (LNQ) q8 = ln_query<NW>(lq, lr, h, sP);
   v4i qv[NQ];
   if constexpr (NQ > 1) {
 #pragma unroll
@@ -1252,10 +1291,11 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_stream_kernel(AttnArgs a,
 // LayerNorm before the cross-attention (one row per block, 20 blocks per
 // row at Whisper-large) and the head's 64 query channels, while the first
 // K chunks are in flight; it replaces a LayerNorm and a query GEMM launch.
-// (five blocks per CU, as the plain kernel: at most 96 VGPRs)
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void attn_decode_cross_lnq_kernel(
-    AttnArgs a, LnQueryArgs lq) {
-  attn_decode_stream_body<2048, IW_DS_NR, IW_DS_CH, 4, false, 1, true>(a, nullptr, lq);
+// (with four waves five blocks per CU, as the plain kernel: at most 96 VGPRs)
+template <int NR, int CH, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4 ? 5 : 4, 8)))
+void attn_decode_cross_lnq_kernel(AttnArgs a, LnQueryArgs lq) {
+  attn_decode_stream_body<2048, NR, CH, NW, false, 1, true>(a, nullptr, lq);
 }
 
 // ---------------------------------------------------------------------------
@@ -1543,7 +1583,12 @@ int launch_attn_decode_cross_lnq(const AttnArgs &a, const LnQueryArgs &lq, hipSt
   if (a.D != 64 || (al & 15) != 0 || a.v_sq != 4 || a.max_tk != a.Tk || a.Tk > 2048 || lq.hidden != a.H * 64 ||
       lq.hidden > 1280 || lq.kp > 1280 || lq.code < 0)
     return fail("the fused cross-attention takes head_dim 64, V transposed, at most 2048 keys and 1280 channels");
-  hipLaunchKernelGGL(attn_decode_cross_lnq_kernel, dim3((unsigned)(a.B * a.H)), dim3(256), 0, s, a, lq);
+  const dim3 grid((unsigned)(a.B * a.H));
+  if (grid.x <= kManyWavesMaxBlocks)
+    hipLaunchKernelGGL((attn_decode_cross_lnq_kernel<DM_NR, DM_CH, DM_NW>), grid, dim3(64 * DM_NW), 0, s,
+                       a, lq);
+  else
+    hipLaunchKernelGGL((attn_decode_cross_lnq_kernel<IW_DS_NR, IW_DS_CH, 4>), grid, dim3(256), 0, s, a, lq);
   return check_launch("attn_decode_cross_lnq_kernel");
 }
 
@@ -1566,6 +1611,9 @@ int launch_attn_decode_cache(const AttnArgs &a, const int32_t *pos, hipStream_t 
   if (a.max_tk <= 512)                                                                                         \
     hipLaunchKernelGGL((attn_decode_stream_kernel<512, IW_DSS_NR, IW_DSS_CH, IW_DSS_NW, VQ_>), grid,            \
                        dim3(64 * IW_DSS_NW), 0, s, a, pos);                                                    \
+  else if (a.max_tk <= 2048 && grid.x <= kManyWavesMaxBlocks)                                                  \
+    hipLaunchKernelGGL((attn_decode_stream_kernel<2048, DM_NR, DM_CH, DM_NW, VQ_>), grid,              \
+                       dim3(64 * DM_NW), 0, s, a, pos);                                                     \
   else if (a.max_tk <= 2048)                                                                                   \
     hipLaunchKernelGGL((attn_decode_stream_kernel<2048, IW_DS_NR, IW_DS_CH, 4, VQ_>), grid, dim3(256), 0, s, a, \
                        pos);                                                                                   \
@@ -1604,7 +1652,14 @@ int launch_attn_decode_cache(const AttnArgs &a, const int32_t *pos, hipStream_t 
     return check_launch("attn_decode_stream_kernel");
   }
   if (vq) return fail("V in key quads needs head_dim 64 and 16-byte aligned operands");
-#define IW_DC(D_, P_) hipLaunchKernelGGL((attn_decode_cache_kernel<D_, P_>), grid, dim3(256), 0, s, a, pos)
+  const bool few = grid.x <= kManyWavesBlocks;
+#define IW_DC(D_, P_)                                                                                    \
+  do {                                                                                                   \
+    if (few)                                                                                             \
+      hipLaunchKernelGGL((attn_decode_cache_kernel<D_, 2, 16>), grid, dim3(1024), 0, s, a, pos);         \
+    else                                                                                                 \
+      hipLaunchKernelGGL((attn_decode_cache_kernel<D_, P_, 4>), grid, dim3(256), 0, s, a, pos);          \
+  } while (0)
   switch (a.D) {
     case 64:
       if (sets <= 1) IW_DC(64, 1); else IW_DC(64, 2);
@@ -1636,15 +1691,22 @@ int launch_attn_decode(const AttnArgs &a, hipStream_t s) {
     c.max_tk = a.Tk;
     c.o_frag_kp = 0;
     const dim3 grid((unsigned)(a.B * a.H));
-#define IW_DQ(NQ_) \
-  hipLaunchKernelGGL((attn_decode_stream_kernel<2048, IW_DS_NR, IW_DS_CH, 4, false, NQ_>), grid, dim3(256), 0, s, c, \
-                     nullptr)
-    if (a.Tq <= 2)
+#define IW_DQ(NQ_)                                                                                                 \
+  if (grid.x <= kManyWavesMaxBlocks)                                                                               \
+    hipLaunchKernelGGL((attn_decode_stream_kernel<2048, DM_NR, DM_CH, DM_NW, false, NQ_>), grid,           \
+                       dim3(64 * DM_NW), 0, s, c, nullptr);                                                     \
+  else                                                                                                             \
+    hipLaunchKernelGGL((attn_decode_stream_kernel<2048, IW_DS_NR, IW_DS_CH, 4, false, NQ_>), grid, dim3(256), 0,   \
+                       s, c, nullptr)
+    if (a.Tq == 1) {
+      IW_DQ(1);
+    } else if (a.Tq <= 2) {
       IW_DQ(2);
-    else if (a.Tq <= 4)
+    } else if (a.Tq <= 4) {
       IW_DQ(4);
-    else
+    } else {
       IW_DQ(8);
+    }
 #undef IW_DQ
     return check_launch("attn_decode_stream_kernel");
   }

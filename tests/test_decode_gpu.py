@@ -405,3 +405,16 @@ def test_fused_cross_attention_does_not_change_results(iw, gpu, tiny_model):
                   for r in eager]
     assert np.array_equal(toks[0], toks[1])
     assert np.array_equal(logits[0], logits[1])
+
+
+# One (batch, head) per CU and fewer take 16 waves per block, more take four:
+# both forms, at the edges of their 256- and 128-key chunks.
+@pytest.mark.parametrize("B,H", [(2, 8), (16, 16), (14, 20)])
+@pytest.mark.parametrize("D,Tk", [(64, 600), (64, 1025), (64, 1500), (96, 17), (96, 1500), (128, 1300)])
+def test_attention_decode_cache_block_counts(iw, oracle, gpu, B, H, D, Tk):
+    test_attention_decode_cache(iw, oracle, gpu, B, H, D, Tk, Tk, 1, "vt")
+
+
+@pytest.mark.parametrize("B,H,Tk", [(1, 6, 1), (1, 8, 255), (20, 12, 257), (12, 20, 1500), (14, 20, 129)])
+def test_attention_decode_cross_lnq_block_counts(iw, oracle, gpu, B, H, Tk):
+    test_attention_decode_cross_lnq(iw, oracle, gpu, B, H, Tk, True, True)

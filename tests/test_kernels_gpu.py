@@ -392,6 +392,14 @@ def test_attention_decode_fused(iw, oracle, gpu, B, H, Tq, Tk, D, masked):
     assert np.array_equal(got, exp)
 
 
+@pytest.mark.parametrize("B,H", [(1, 5), (16, 16), (19, 14)])
+@pytest.mark.parametrize("Tq,Tk", [(1, 1), (1, 1500), (2, 256), (3, 257), (8, 1030)])
+def test_attention_decode_block_counts(iw, oracle, gpu, B, H, Tq, Tk):
+    """Query rows sharing a stream on both sides of one block per CU (16 and 4
+    waves per block)."""
+    test_attention_decode_fused(iw, oracle, gpu, B, H, Tq, Tk, 64, False)
+
+
 @pytest.mark.parametrize("decode", [False, True])
 def test_attention_fused_wrap_corner(iw, oracle, gpu, decode):
     """Scores saturating at +32767 wrap rmp1 and give P = 128 at x_sub = 0."""
