@@ -573,14 +573,27 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return v;
 }
 
-__global__ __launch_bounds__(256) void greedy_filtered_kernel(const int8_t *__restrict__ x, int64_t cols,
-                                                              int64_t ld, int64_t *__restrict__ out,
-                                                              int64_t *__restrict__ history, int64_t hist_ld,
-                                                              int64_t hist_cols, const int32_t *step,
-                                                              GreedyFilter f) {
-  __shared__ uint32_t s_kt[4], s_ks[4];
-  __shared__ int32_t s_m[4], s_i[4], s_mx[4];
-  __shared__ float s_s[4], s_sx[4];
+// The elements e of [i0, i0 + 16) with lo <= i0 + e < hi, as bits.
+__device__ __forceinline__ uint32_t range_bits16(int i0, int lo, int hi) {
+  const int a = min(max(lo - i0, 0), 16), b = min(max(hi - i0, 0), 16);
+  return ((1u << b) - 1u) & ~((1u << a) - 1u);
+}
+
+// A row is one block's, so the time is that of its chain: 1024 threads read the
+// row in 16-byte pieces twice, for the maxima and then for the sums of
+// exp((x - max) scale) from a 256-entry table in LDS (one expf per value
+// instead of one per logit). A pass of 256 threads, a byte and an expf at a
+// time, took 62.6 us per step for 27 rows of 51865 logits; this takes 12.
+constexpr int GF_NT = 1024, GF_NW = GF_NT / 64;
+
+__global__ __launch_bounds__(GF_NT) void greedy_filtered_kernel(const int8_t *__restrict__ x, int64_t cols,
+                                                                int64_t ld, int64_t *__restrict__ out,
+                                                                int64_t *__restrict__ history, int64_t hist_ld,
+                                                                int64_t hist_cols, const int32_t *step,
+                                                                GreedyFilter f) {
+  __shared__ uint32_t s_kt[GF_NW], s_ks[GF_NW];
+  __shared__ int32_t s_i[GF_NW];
+  __shared__ float s_s[GF_NW], s_sx[GF_NW], s_et[256], s_ex[256];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t row = blockIdx.x;
   const int n = (int)cols;
@@ -605,12 +618,13 @@ __global__ __launch_bounds__(256) void greedy_filtered_kernel(const int8_t *__re
     }
     // the last timestamp sampled so far
     int im = -1;
-    for (int i = tid; i < nh; i += 256)
+    for (int i = tid; i < nh; i += GF_NT)
       if (h[i] >= f.ts_begin) im = i;
     im = wave_max_i32(im);
     if (lane == 0) s_i[wave] = im;
     __syncthreads();
-    im = max(max(s_i[0], s_i[1]), max(s_i[2], s_i[3]));
+#pragma unroll
+    for (int w = 0; w < GF_NW; ++w) im = max(im, s_i[w]);
     if (im >= 0) {
       const int64_t tl = h[im] + ((last_ts && !pen_ts) ? 0 : 1);  // non-decreasing, nonzero segments
       ts_lo = (int)min(max((int64_t)ts_lo, tl), (int64_t)n);
@@ -624,75 +638,87 @@ __global__ __launch_bounds__(256) void greedy_filtered_kernel(const int8_t *__re
   const uint32_t *mk = (st == 0 && f.mask_first) ? f.mask_first : f.mask;
   const int nw = (n + 31) >> 5;
 
-  // ---- one pass: text argmax key, timestamp argmax key, timestamp (max, sum exp),
-  // and with sum_logprobs the text tokens' (max, sum exp) ----
-  const bool lps = f.sum_logprobs != nullptr;
-  uint32_t kt = 0, ks = 0;
-  int32_t m = -1000, mx = -1000;
-  float sum = 0.f, sumx = 0.f;
+  // visit(g): g(i0, words, text, ts) for pieces of up to 16 consecutive logits
+  // from i0, with the allowed text and timestamp elements as bits
   const int8_t *xr = x + row * ld;
-  for (int i0 = tid * 16; i0 < n; i0 += 256 * 16) {
-    uint32_t bits = 0;
+  const int head = min((int)((16 - (reinterpret_cast<uintptr_t>(xr) & 15)) & 15), n);
+  const int pieces = (n - head) >> 4, tail0 = head + (pieces << 4);
+  auto piece = [&](int i0, uint4 w, uint32_t in, auto &&g) {
     if (mk) {
-      const int w = i0 >> 5, sh = i0 & 31;
-      uint64_t pair = mk[w];
-      if (w + 1 < nw) pair |= (uint64_t)mk[w + 1] << 32;
-      bits = (uint32_t)(pair >> sh) & 0xffffu;
+      const int k = i0 >> 5;
+      uint64_t pair = mk[k];
+      if (k + 1 < nw) pair |= (uint64_t)mk[k + 1] << 32;
+      in &= ~(uint32_t)(pair >> (i0 & 31));
     }
-#pragma unroll 4
+    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+    g(i0, ws, in & range_bits16(i0, text_lo, ts_b), in & range_bits16(i0, ts_lo, ts_hi));
+  };
+  auto visit = [&](auto &&g) {
+    if (tid < head) piece(tid, make_uint4((uint8_t)xr[tid], 0, 0, 0), 1u, g);
+    for (int c = tid; c < pieces; c += GF_NT)
+      piece(head + (c << 4), *reinterpret_cast<const uint4 *>(xr + head + (c << 4)), 0xffffu, g);
+    if (tail0 + tid < n) piece(tail0 + tid, make_uint4((uint8_t)xr[tail0 + tid], 0, 0, 0), 1u, g);
+  };
+  auto value = [](const uint32_t (&ws)[4], int e) { return (int32_t)(int8_t)(ws[e >> 2] >> (8 * (e & 3))); };
+
+  // ---- text and timestamp argmax keys ----
+  uint32_t kt = 0, ks = 0;
+  visit([&](int i0, const uint32_t (&ws)[4], uint32_t tb, uint32_t sb) {
+#pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int i = i0 + e;
-      if (i >= n || ((bits >> e) & 1)) continue;
-      const int32_t v = xr[i];
-      const uint32_t key = ((uint32_t)(v + 129) << 23) | (uint32_t)(0x7FFFFF - i);
-      if (i >= text_lo && i < ts_b) {
-        kt = max(kt, key);
-        if (lps) {
-          if (v > mx) {
-            sumx = sumx * expf((float)(mx - v) * f.scale) + 1.f;
-            mx = v;
-          } else {
-            sumx += expf((float)(v - mx) * f.scale);
-          }
-        }
-      } else if (i >= ts_lo && i < ts_hi) {
-        ks = max(ks, key);
-        if (v > m) {
-          sum = sum * expf((float)(m - v) * f.scale) + 1.f;
-          m = v;
-        } else {
-          sum += expf((float)(v - m) * f.scale);
-        }
-      }
+      const uint32_t key = ((uint32_t)(value(ws, e) + 129) << 23) | (uint32_t)(0x7FFFFF - (i0 + e));
+      if ((tb >> e) & 1u) kt = max(kt, key);
+      if ((sb >> e) & 1u) ks = max(ks, key);
     }
-  }
+  });
   kt = wave_max_u32(kt);
   ks = wave_max_u32(ks);
-  int32_t mw = wave_max_i32(m);
-  float sw = sum * expf((float)(m - mw) * f.scale);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) sw += __shfl_xor(sw, o);
-  if (lane == 0) s_kt[wave] = kt, s_ks[wave] = ks, s_m[wave] = mw, s_s[wave] = sw;
-  if (lps) {
-    const int32_t mxw = wave_max_i32(mx);
-    float sxw = sumx * expf((float)(mx - mxw) * f.scale);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) sxw += __shfl_xor(sxw, o);
-    if (lane == 0) s_mx[wave] = mxw, s_sx[wave] = sxw;
-  }
+  if (lane == 0) s_kt[wave] = kt, s_ks[wave] = ks;
   __syncthreads();
+#pragma unroll
+  for (int w = 0; w < GF_NW; ++w) kt = max(kt, s_kt[w]), ks = max(ks, s_ks[w]);
+  const int32_t mt = (int32_t)(ks >> 23) - 129, mxt = (int32_t)(kt >> 23) - 129;  // the two maxima
+
+  // ---- sums of exp((x - max) scale) over the allowed timestamps, and with
+  // sum_logprobs over the allowed text ----
+  const bool lps = f.sum_logprobs != nullptr;
+  float st_sum = 0.f, sx = 0.f;
+  if (lps || (rules && ks != 0)) {
+    if (tid < 256) {
+      s_et[tid] = expf((float)(tid - 128 - mt) * f.scale);
+      s_ex[tid] = expf((float)(tid - 128 - mxt) * f.scale);
+    }
+    __syncthreads();
+    visit([&](int, const uint32_t (&ws)[4], uint32_t tb, uint32_t sb) {
+      if (lps && tb) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float p = s_ex[value(ws, e) + 128];
+          if ((tb >> e) & 1u) sx += p;
+        }
+      }
+      if (sb) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float p = s_et[value(ws, e) + 128];
+          if ((sb >> e) & 1u) st_sum += p;
+        }
+      }
+    });
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) st_sum += __shfl_xor(st_sum, o), sx += __shfl_xor(sx, o);
+    if (lane == 0) s_s[wave] = st_sum, s_sx[wave] = sx;
+    __syncthreads();
+  }
   if (tid == 0) {
-    kt = max(max(s_kt[0], s_kt[1]), max(s_kt[2], s_kt[3]));
-    ks = max(max(s_ks[0], s_ks[1]), max(s_ks[2], s_ks[3]));
     uint32_t key = max(kt, ks);
-    // the timestamps' (max, sum exp) over the allowed timestamps
-    const int32_t mt = max(max(s_m[0], s_m[1]), max(s_m[2], s_m[3]));
-    float st_sum = 0.f;
-    for (int w = 0; w < 4; ++w) st_sum += s_s[w] * expf((float)(s_m[w] - mt) * f.scale);
+    st_sum = sx = 0.f;
+    if (lps || (rules && ks != 0))
+      for (int w = 0; w < GF_NW; ++w) st_sum += s_s[w], sx += s_sx[w];
     bool ts_wins = false;
     if (rules && ks != 0) {
       const float lse_ts = (float)mt * f.scale + logf(st_sum);
-      ts_wins = kt == 0 || lse_ts > (float)((int32_t)(kt >> 23) - 129) * f.scale;
+      ts_wins = kt == 0 || lse_ts > (float)mxt * f.scale;
       if (ts_wins) key = ks;
     }
     int64_t idx = key == 0 ? 0 : (int64_t)(0x7FFFFF - (key & 0x7FFFFF));
@@ -712,9 +738,6 @@ __global__ __launch_bounds__(256) void greedy_filtered_kernel(const int8_t *__re
       } else if (ts_wins || kt == 0) {
         lp = -logf(st_sum);
       } else {
-        const int32_t mxt = max(max(s_mx[0], s_mx[1]), max(s_mx[2], s_mx[3]));
-        float sx = 0.f;
-        for (int w = 0; w < 4; ++w) sx += s_sx[w] * expf((float)(s_mx[w] - mxt) * f.scale);
         const int32_t top = (int32_t)(key >> 23) - 129;  // the chosen value
         float total = sx * expf((float)(mxt - top) * f.scale);
         if (ks != 0) total += st_sum * expf((float)(mt - top) * f.scale);
@@ -1184,7 +1207,7 @@ int launch_greedy_step_filtered(const int8_t *logits, int64_t rows, int64_t cols
                                 float scale, float *sum_logprobs, int32_t *eot_count, hipStream_t s) {
   if (rows > 0) {
     const GreedyFilter f{mask, mask_first, prev0, eot, ts_begin, max_init, scale, sum_logprobs, eot_count};
-    hipLaunchKernelGGL(greedy_filtered_kernel, dim3((unsigned)rows), dim3(256), 0, s, logits, cols, ld, next,
+    hipLaunchKernelGGL(greedy_filtered_kernel, dim3((unsigned)rows), dim3(GF_NT), 0, s, logits, cols, ld, next,
                        history, hist_ld, hist_cols, step, f);
     int rc = check_launch("greedy_filtered_kernel");
     if (rc) return rc;
