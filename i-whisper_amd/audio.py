@@ -125,5 +125,5 @@ def log_mel_spectrogram(audio: torch.Tensor, n_mels: int = 80, padding: int = 0,
     ws = torch.empty(B * ((T + 63) // 64), dtype=torch.float32, device=a.device)
     _lib.call("iw_log_mel", a.data_ptr(), B, L, L, fe.twiddle.data_ptr(), fe.window.data_ptr(),
               fe.start.data_ptr(), fe.len.data_ptr(), fe.off.data_ptr(), fe.w.data_ptr(), fe.n_taps, n_mels,
-              out.data_ptr(), n_mels * T, ws.data_ptr(), torch.cuda.current_stream().cuda_stream)
+              out.data_ptr(), n_mels * T, ws.data_ptr(), _lib.stream())
     return out[0] if single else out

@@ -19,8 +19,7 @@ from . import _lib
 Tensor = torch.Tensor
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.stream
 
 
 def _check(t: Tensor, dtype: torch.dtype, name: str) -> None:

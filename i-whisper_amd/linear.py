@@ -22,8 +22,7 @@ from . import _lib
 BACKENDS = ("hip",)
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.stream
 
 
 def check_backend(backend: str) -> None:
@@ -67,11 +66,14 @@ class LinearBase(nn.Linear):
         if x.size(-1) != K:
             raise RuntimeError(f"weight.size(1) must equal x.size(-1), expected {x.size(-1)}, got {K}")
         M = x.numel() // K
-        b = self.bias
+        try:  # nn.Module's attribute lookups cost more than the pointers
+            p = self._parameters
+            w, b, m, s = p["weight"], p["bias"], p["req_multiplier"], p["req_shiftmount"]
+        except KeyError:  # parametrized and replicated modules hold them elsewhere
+            w, b, m, s = self.weight, self.bias, self.req_multiplier, self.req_shiftmount
         z = self.wgt_zeros if self.asym else None
-        return x, M, (self.weight.data_ptr(), None if b is None else b.data_ptr(),
-                      None if z is None else z.data_ptr(), self.req_multiplier.data_ptr(),
-                      self.req_shiftmount.data_ptr())
+        return x, M, (w.data_ptr(), None if b is None else b.data_ptr(),
+                      None if z is None else z.data_ptr(), m.data_ptr(), s.data_ptr())
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         raise NotImplementedError("Use Linear8 or Linear32")

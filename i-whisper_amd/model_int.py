@@ -33,8 +33,7 @@ __all__ = [
 ]
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.stream
 
 
 def _ptr(t: Optional[Tensor]) -> Optional[int]:
@@ -114,10 +113,9 @@ class GELU_int(nn.Module):
                                           requires_grad=False)
 
     def gelu_ptrs(self):
-        return (self.lut.data_ptr(), self.luti_req_multiplier.data_ptr(),
-                self.luti_req_shiftmount.data_ptr(), self.luto_req_multiplier.data_ptr(),
-                self.luto_req_shiftmount.data_ptr(), self.luti_req_multiplier.numel(),
-                self.luto_req_multiplier.numel())
+        im, om = self.luti_req_multiplier, self.luto_req_multiplier
+        return (self.lut.data_ptr(), im.data_ptr(), self.luti_req_shiftmount.data_ptr(), om.data_ptr(),
+                self.luto_req_shiftmount.data_ptr(), im.numel(), om.numel())
 
     def forward(self, x: Tensor) -> Tensor:
         assert x.dtype == torch.int8, "Input tensor must be int8 in integer inference mode!"
@@ -611,8 +609,10 @@ class TextDecoder_int(nn.Module):
     def forward(self, x: Tensor, xa: Tensor, kv_cache: Optional[dict] = None):
         check_backend(self.backend)
         offset = next(iter(kv_cache.values())).shape[1] if kv_cache else 0
-        if x.numel() and (int(x.min()) < 0 or int(x.max()) >= self.n_vocab):
-            raise RuntimeError("token id out of range")
+        if x.numel():
+            lo, hi = torch.stack(torch.aminmax(x)).tolist()  # one read of the device
+            if lo < 0 or hi >= self.n_vocab:
+                raise RuntimeError("token id out of range")
         x = self.embed(x, offset)
         for block in self.blocks:
             x = block(x, xa, mask=self.mask, kv_cache=kv_cache)

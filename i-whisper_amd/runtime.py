@@ -36,8 +36,7 @@ from . import _lib
 from .model_int import AudioEncoder_int, ResidualAttentionBlock_int, TextDecoder_int, Whisper_int
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.stream
 
 
 def _ptr(t):

@@ -10,8 +10,7 @@ import torch
 from . import _lib
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.stream
 
 
 def median_filter(x: torch.Tensor, filter_width: int) -> torch.Tensor:
