@@ -153,6 +153,40 @@ def test_conv1d_channels_last_big(iw, oracle, gpu, B, Cin, Tin, Cout, stride):
     assert np.array_equal(host(out16), exp16)
 
 
+# Convolutions over the direct-to-LDS tiles: one position, rows without any tap
+# inside the input, K of no whole stage, ragged rows and columns, sequences that
+# end inside a tile, each tile size, GeLU as a table and per channel.
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("B,Cin,Tin,Cout,ks,stride,pad", [
+    (1, 16, 1, 16, 1, 1, 0), (2, 32, 40, 64, 5, 3, 7), (5, 80, 333, 384, 3, 1, 1), (7, 48, 61, 80, 3, 2, 1),
+    (1, 384, 3000, 384, 3, 2, 1), (2, 512, 2999, 1040, 3, 2, 1), (5, 128, 3000, 1024, 3, 1, 1),
+    (17, 80, 1501, 1296, 3, 1, 1)])
+def test_conv1d_channels_last_tiles(iw, oracle, gpu, B, Cin, Tin, Cout, ks, stride, pad, per_channel):
+    print("case: conv1d_cl tiles", B, Cin, Tin, Cout, ks, stride, pad, per_channel, flush=True)
+    r = gen.rng(B * Cin + Tin + Cout + ks)
+    x = gen.i8(r, (B, Cin, Tin))
+    w = gen.i8(r, (Cout, Cin * ks), -60, 60)
+    bias = r.integers(-2**16, 2**16, size=Cout).astype(np.int32)
+    mult, shift = int(r.integers(2**29, 2**31)), 9
+    lut, im, is_, om, os_ = gen.gelu_params(r, Cout, False, per_channel)
+    conv = oracle.conv1d(x, w, bias, mult, shift, stride, pad)
+    g = oracle.gelu(np.ascontiguousarray(conv.transpose(0, 2, 1)), lut, im, is_, om, os_)
+    tout = g.shape[1]
+    pe = gen.i8(r, (tout, Cout))
+    pm = r.integers(1, 65536, size=Cout if per_channel else 1).astype(np.uint16)
+    ps = r.integers(-1, 33, size=Cout).astype(np.int8)
+    exp16 = oracle.add_requant15(g, pe, pm, ps)
+    ts = [T(np.ascontiguousarray(x.transpose(0, 2, 1))), T(_kc(w, Cin, ks)), T(bias)]
+    gt = [T(a) for a in (lut, im, is_, om, os_)]
+    pt = [T(a) for a in (pe, pm, ps)]
+    for pos, exp in ((False, g), (True, exp16)):
+        out = torch.empty(exp.shape, dtype=torch.int16 if pos else torch.int8, device="cuda")
+        iw._lib.call("iw_conv1d_cl", *(t.data_ptr() for t in ts), mult, shift, *(t.data_ptr() for t in gt), len(im),
+                     len(om), *(t.data_ptr() if pos else None for t in pt), len(pm) if pos else 0,
+                     len(ps) if pos else 0, out.data_ptr(), B, Cin, Tin, Cout, ks, stride, pad, True, stream())
+        assert np.array_equal(host(out), exp)
+
+
 # The direct-to-LDS GEMM (K % 64 == 0, N % 16 == 0) at shapes with several
 # times more 256 x 256 tiles than the GPU has CUs, ragged M (and N) edges,
 # in-place residual, per-tensor GeLU (the table form) and multipliers on both
