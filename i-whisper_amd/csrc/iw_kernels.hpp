@@ -67,7 +67,9 @@ struct LnQueryArgs {
   const int8_t *shift = nullptr;
 };
 
-int layernorm_width_code(int64_t h);
+constexpr int layernorm_width_code(int64_t h) {
+  return h == 384 ? 0 : h == 512 ? 1 : h == 768 ? 2 : h == 1024 ? 3 : h == 1280 ? 4 : -1;
+}
 // out_frag: out is the fragment-major image of [rows][hidden] (rows <= 128)
 int launch_layernorm32(const int16_t *x, const int8_t *gamma, const int32_t *beta, uint8_t ln_m,
                        int8_t ln_s, uint32_t out_m, int8_t out_s, uint32_t rsqrt_off, int8_t *out,

@@ -2,6 +2,8 @@
 // residual15, add_requant15, token-embedding gather, log-mel quantization and
 // the greedy argmax. All are HBM-bound; each reads and writes its operands
 // once.
+#include <type_traits>
+
 #include "iw_common.hpp"
 #include "iw_gemm.hpp"
 #include "iw_kernels.hpp"
@@ -28,7 +30,10 @@ typedef short s16x2 __attribute__((ext_vector_type(2)));
 // The row lives in registers: lane l owns 4-element chunks l, l + 64, ...
 // The waves are persistent: each loads its lanes' gamma / beta once, then
 // walks the rows wave_id, wave_id + waves, ..., requesting the next row
-// before reducing the current one.
+// before reducing the current one. One instance per width, so that a narrow row
+// has neither the registers nor the chunk tests of a wide one: more waves per
+// SIMD to hide the chain of reductions that every row has (192000 rows of 512
+// columns 115 -> 83 us, of 1024 160 -> 147, of 1280 183 -> 179).
 //
 // The integer steps are the reference's; their arithmetic is arranged for
 // the VALU, which bounds this kernel at encoder sizes:
@@ -43,34 +48,33 @@ typedef short s16x2 __attribute__((ext_vector_type(2)));
 //   formed once per row (written as two 24-bit products, which the compiler
 //   may fuse back into one 32-bit multiply), and mulh is a signed high
 //   multiply with a mask correction for multipliers >= 2^31.
-constexpr int LN_MAX_CHUNKS = 5;  // 1280 / 4 / 64
-
+template <int HIDDEN>
 __global__ __launch_bounds__(256) void layernorm32_kernel(
     const int16_t *__restrict__ x, const int8_t *__restrict__ gamma,
     const int32_t *__restrict__ beta, uint32_t ln_m, int32_t ln_s, uint32_t out_m,
-    int32_t out_s, uint32_t rsqrt_off, int8_t *__restrict__ out, int64_t rows, int hidden,
-    int code) {
+    int32_t out_s, uint32_t rsqrt_off, int8_t *__restrict__ out, int64_t rows) {
+  constexpr int hidden = HIDDEN, code = layernorm_width_code(HIDDEN);
+  constexpr int nch = HIDDEN / 4, NCH = (nch + 63) / 64;  // >= 96: every lane owns chunk 0
   const int lane = threadIdx.x & 63;
   const int64_t wave_id = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
   if (wave_id >= rows) return;
-  const int nch = hidden >> 2;  // >= 96: every lane owns chunk 0
   auto load_row = [&](int64_t r, uint2 *w) {
     const int16_t *xr = x + r * hidden;
 #pragma unroll
-    for (int c = 0; c < LN_MAX_CHUNKS; ++c) {
+    for (int c = 0; c < NCH; ++c) {
       const int ch = lane + 64 * c;
       w[c] = ch < nch ? *reinterpret_cast<const uint2 *>(xr + ch * 4) : make_uint2(0, 0);
     }
   };
-  uint2 xa[LN_MAX_CHUNKS];
+  uint2 xa[NCH];
   load_row(wave_id, xa);
   const bool g_al = (reinterpret_cast<uintptr_t>(gamma) & 3) == 0;
   const bool b_al = beta && (reinterpret_cast<uintptr_t>(beta) & 15) == 0;
-  uint32_t gw[LN_MAX_CHUNKS];
-  uint4 bw[LN_MAX_CHUNKS];
+  uint32_t gw[NCH];
+  uint4 bw[NCH];
 #pragma unroll
-  for (int c = 0; c < LN_MAX_CHUNKS; ++c) {
+  for (int c = 0; c < NCH; ++c) {
     const int ch = lane + 64 * c;
     gw[c] = 0;
     bw[c] = make_uint4(0, 0, 0, 0);
@@ -93,15 +97,14 @@ __global__ __launch_bounds__(256) void layernorm32_kernel(
   const bool out_zero = (uint32_t)out_s >= 32;
   const uint32_t om = out_zero ? 0u : out_m;
   const uint32_t osh = out_zero ? 0u : (uint32_t)out_s;
-  const uint32_t omneg = (uint32_t)((int32_t)om >> 31);
   const s16x2 ones = {1, 1};
   // one row: xw holds its raw values on entry and is refilled with row
   // `next` (if any) as soon as they are unpacked
-  auto process = [&](int64_t row, uint2 *xw, int64_t next) {
+  auto process = [&](int64_t row, uint2 *xw, int64_t next, auto big) {
     int32_t sum = 0;
     s16x2 mx2 = {-32768, -32768}, mn2 = {32767, 32767};
 #pragma unroll
-    for (int c = 0; c < LN_MAX_CHUNKS; ++c) {
+    for (int c = 0; c < NCH; ++c) {
       if (lane + 64 * c < nch) {
         const s16x2 p0 = __builtin_bit_cast(s16x2, xw[c].x), p1 = __builtin_bit_cast(s16x2, xw[c].y);
         sum = __builtin_amdgcn_sdot2(p0, ones, sum, false);
@@ -110,9 +113,9 @@ __global__ __launch_bounds__(256) void layernorm32_kernel(
         mn2 = __builtin_elementwise_min(mn2, __builtin_elementwise_min(p0, p1));
       }
     }
-    int32_t v[LN_MAX_CHUNKS][4];
+    int32_t v[NCH][4];
 #pragma unroll
-    for (int c = 0; c < LN_MAX_CHUNKS; ++c) {
+    for (int c = 0; c < NCH; ++c) {
       v[c][0] = (int16_t)(xw[c].x & 0xffff);
       v[c][1] = (int16_t)(xw[c].x >> 16);
       v[c][2] = (int16_t)(xw[c].y & 0xffff);
@@ -124,7 +127,7 @@ __global__ __launch_bounds__(256) void layernorm32_kernel(
     const int32_t xmin = -wave_max_dpp(-min((int32_t)mn2.x, (int32_t)mn2.y));
     const int32_t mean = norm_reduce(total, code);
 #pragma unroll
-    for (int c = 0; c < LN_MAX_CHUNKS; ++c)
+    for (int c = 0; c < NCH; ++c)
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[c][e] -= mean;  // d
     const int32_t maxabs = max(xmax - mean, mean - xmin);
@@ -135,7 +138,7 @@ __global__ __launch_bounds__(256) void layernorm32_kernel(
     } else {
       maxsq = 0;
 #pragma unroll
-      for (int c = 0; c < LN_MAX_CHUNKS; ++c)
+      for (int c = 0; c < NCH; ++c)
         if (lane + 64 * c < nch)
 #pragma unroll
           for (int e = 0; e < 4; ++e) maxsq = max(maxsq, (int32_t)((uint32_t)v[c][e] * (uint32_t)v[c][e]));
@@ -149,13 +152,13 @@ __global__ __launch_bounds__(256) void layernorm32_kernel(
       // d^2 < 2^31 and rs <= 16: rshift of a non-negative value, no wrap
       const int32_t half = rs ? 1 << (rs - 1) : 0;
 #pragma unroll
-      for (int c = 0; c < LN_MAX_CHUNKS; ++c)
+      for (int c = 0; c < NCH; ++c)
         if (lane + 64 * c < nch)
 #pragma unroll
           for (int e = 0; e < 4; ++e) vs += (uint32_t)(__mul24(v[c][e], v[c][e]) + half) >> rs;
     } else {
 #pragma unroll
-      for (int c = 0; c < LN_MAX_CHUNKS; ++c)
+      for (int c = 0; c < NCH; ++c)
         if (lane + 64 * c < nch)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -172,7 +175,7 @@ __global__ __launch_bounds__(256) void layernorm32_kernel(
     const uint32_t ohalf = osh ? 1u << (osh - 1) : 0u, ow = min(osh, 1u);
     int8_t *orow = out + row * hidden;
 #pragma unroll
-    for (int c = 0; c < LN_MAX_CHUNKS; ++c) {
+    for (int c = 0; c < NCH; ++c) {
       const int ch = lane + 64 * c;
       if (ch < nch) {
         uint32_t packed = 0;
@@ -185,7 +188,7 @@ __global__ __launch_bounds__(256) void layernorm32_kernel(
           const int32_t y = clampi((int32_t)(t + nhalf + ts) >> nshift, -16383, 16383);
           const uint32_t a = (uint32_t)__mul24(y, (int32_t)(int8_t)(gw[c] >> (8 * e))) + bv[e];
           // mulh(a, om): signed high word, plus a when om >= 2^31
-          const uint32_t hi = (uint32_t)__mulhi((int32_t)a, (int32_t)om) + (a & omneg);
+          const uint32_t hi = (uint32_t)__mulhi((int32_t)a, (int32_t)om) + (decltype(big)::value ? a : 0u);
           const uint32_t hs = (uint32_t)__builtin_amdgcn_sbfe((int32_t)hi, 31, ow);
           const int32_t o = clampi((int32_t)(hi + ohalf + hs) >> osh, -127, 127);
           packed |= ((uint32_t)(uint8_t)(int8_t)o) << (8 * e);
@@ -195,7 +198,11 @@ __global__ __launch_bounds__(256) void layernorm32_kernel(
     }
   };
   // rows wave_id + k * waves, the next one in flight
-  for (int64_t row = wave_id; row < rows; row += waves) process(row, xa, row + waves);
+  if ((int32_t)om < 0) {
+    for (int64_t row = wave_id; row < rows; row += waves) process(row, xa, row + waves, std::true_type{});
+  } else {
+    for (int64_t row = wave_id; row < rows; row += waves) process(row, xa, row + waves, std::false_type{});
+  }
 }
 
 // LayerNorm32 for few rows (a decode step): one row per block of 256 threads,
@@ -1031,17 +1038,21 @@ int grid_for(int64_t n, int threads) {
 
 }  // namespace
 
-// row counts up to which each row gets a block of its own
-constexpr int64_t kLnRowBlockMaxRows = 2048;
+// Row counts up to which each row gets a block of its own. Wave rows and block
+// rows take, us: 1500 rows of 384 3.4 / 5.5, of 1280 4.8 / 6.2; 300 of 1280 3.5 / 4.0; at
+// 60 rows block rows are 0.3 ahead at 1280 columns, and only they prefetch the
+// decode GEMMs' weights (at most 128 rows).
+constexpr int64_t kLnRowBlockMaxRows = 256;
 
 // Blocks of layernorm32_kernel resident on the whole device at once (its
 // persistent grid): CUs x blocks per CU at the kernel's register use.
+template <int HIDDEN>
 int64_t ln_persistent_blocks() {
   static const int64_t blocks = [] {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, layernorm32_kernel, 256, 0) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, layernorm32_kernel<HIDDEN>, 256, 0) != hipSuccess ||
         cus <= 0 || per_cu <= 0) {
       (void)hipGetLastError();
       return (int64_t)256 * 4;
@@ -1051,15 +1062,13 @@ int64_t ln_persistent_blocks() {
   return blocks;
 }
 
-int layernorm_width_code(int64_t h) {
-  switch (h) {
-    case 384: return 0;
-    case 512: return 1;
-    case 768: return 2;
-    case 1024: return 3;
-    case 1280: return 4;
-    default: return -1;
-  }
+template <int HIDDEN>
+void launch_layernorm32_waves(const int16_t *x, const int8_t *gamma, const int32_t *beta, uint32_t ln_m, int32_t ln_s,
+                              uint32_t out_m, int32_t out_s, uint32_t rsqrt_off, int8_t *out, int64_t rows,
+                              hipStream_t s) {
+  const int64_t blocks = std::min<int64_t>((rows + 3) / 4, ln_persistent_blocks<HIDDEN>());
+  hipLaunchKernelGGL(layernorm32_kernel<HIDDEN>, dim3((unsigned)blocks), dim3(256), 0, s, x, gamma, beta, ln_m, ln_s,
+                     out_m, out_s, rsqrt_off, out, rows);
 }
 
 int launch_layernorm32(const int16_t *x, const int8_t *gamma, const int32_t *beta, uint8_t ln_m,
@@ -1080,10 +1089,12 @@ int launch_layernorm32(const int16_t *x, const int8_t *gamma, const int32_t *bet
   }
   // one row per wave at a time, four waves per block; persistent waves, as
   // many blocks as the device holds at once
-  const int64_t blocks = std::min<int64_t>((rows + 3) / 4, ln_persistent_blocks());
-  hipLaunchKernelGGL(layernorm32_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, gamma, beta,
-                     (uint32_t)ln_m, (int32_t)ln_s, out_m, (int32_t)out_s, rsqrt_off, out, rows,
-                     (int)hidden, code);
+  const auto waves = code == 0   ? launch_layernorm32_waves<384>
+                     : code == 1 ? launch_layernorm32_waves<512>
+                     : code == 2 ? launch_layernorm32_waves<768>
+                     : code == 3 ? launch_layernorm32_waves<1024>
+                                 : launch_layernorm32_waves<1280>;
+  waves(x, gamma, beta, ln_m, ln_s, out_m, out_s, rsqrt_off, out, rows, s);
   return check_launch("layernorm32_kernel");
 }
 
