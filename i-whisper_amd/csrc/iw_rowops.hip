@@ -997,6 +997,65 @@ __global__ __launch_bounds__(256) void transpose_heads16_kernel(
   }
 }
 
+// The same on 128 x 128 tiles: whole 128-byte lines on both sides and a fourth of
+// the blocks. A thread takes 16 columns of four positions, turns them into 16
+// words of one column's four positions (byte permutes) and writes these to LDS as
+// [column][position], 16-byte groups at group ^ (column / 16) so that a wave's
+// writes spread over the banks. Each XCD takes a run of tiles, positions
+// first: rows of positions start at any 16 bytes, so neighbouring tiles share lines,
+// which one L2 then completes (in the dispatcher's order 175 us at 128 x 1500 x 1280).
+constexpr int TH_T = 128, TH_C = 128;
+__global__ __launch_bounds__(256) void transpose_heads128_kernel(
+    const int8_t *__restrict__ src, int64_t src_sb, int64_t src_st, int8_t *__restrict__ dst, int64_t dst_sb,
+    int64_t dst_sh, int64_t dst_sd, int64_t t_off, int64_t T, int64_t H, int64_t D, uint32_t tiles_t, uint32_t tiles_c,
+    uint32_t tiles, uint32_t per_xcd) {
+  __shared__ __attribute__((aligned(16))) uint32_t tile[TH_C * TH_T / 4];
+  const uint32_t id = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (id >= tiles) return;
+  const uint32_t bc = id / tiles_t;
+  const int64_t b = bc / tiles_c, t0 = (int64_t)(id - bc * tiles_t) * TH_T, c0 = (int64_t)(bc % tiles_c) * TH_C, C = H * D;
+  const int tid = threadIdx.x, tq = tid >> 3, cq = tid & 7;
+  uint4 v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int64_t t = t0 + 4 * tq + i, c = c0 + 16 * cq;
+    v[i] = make_uint4(0, 0, 0, 0);
+    if (t < T && c < C) v[i] = *reinterpret_cast<const uint4 *>(src + b * src_sb + t * src_st + c);
+  }
+  const int pos = ((tq >> 2) ^ cq) * 4 + (tq & 3);
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    auto word = [&](int i) { return w == 0 ? v[i].x : w == 1 ? v[i].y : w == 2 ? v[i].z : v[i].w; };
+    const uint32_t lo01 = __builtin_amdgcn_perm(word(1), word(0), 0x05010400u);
+    const uint32_t hi01 = __builtin_amdgcn_perm(word(1), word(0), 0x07030602u);
+    const uint32_t lo23 = __builtin_amdgcn_perm(word(3), word(2), 0x05010400u);
+    const uint32_t hi23 = __builtin_amdgcn_perm(word(3), word(2), 0x07030602u);
+    uint32_t *o = &tile[(16 * cq + 4 * w) * (TH_T / 4) + pos];
+    o[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+    o[TH_T / 4] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+    o[2 * TH_T / 4] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+    o[3 * TH_T / 4] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+  }
+  __syncthreads();
+  const int g = tid & 7;
+  const int64_t t = t0 + 16 * g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int cl = (tid >> 3) + 32 * i;
+    const int64_t c = c0 + cl;
+    if (c >= C || t >= T) continue;
+    const uint4 w = *reinterpret_cast<const uint4 *>(&tile[cl * (TH_T / 4) + (g ^ (cl >> 4)) * 4]);
+    const int32_t h = (int32_t)c / (int32_t)D, d = (int32_t)c - h * (int32_t)D;
+    int8_t *o = dst + b * dst_sb + (int64_t)h * dst_sh + (int64_t)d * dst_sd + t_off + t;
+    if (t + 16 <= T) {
+      *reinterpret_cast<uint4 *>(o) = w;
+    } else {
+      const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+      for (int e = 0; e < 16 && t + e < T; ++e) o[e] = (int8_t)(ws[e >> 2] >> (8 * (e & 3)));
+    }
+  }
+}
+
 // Per-head gather of a [B, T, H*D] operand slice into a [B, H, T_cap, D]
 // cache at positions [t_off, t_off + T): dst[b*dst_sb + h*dst_sh + (t_off+t)*dst_st + d]
 // = src[b*src_sb + t*src_st + h*D + d], 16 bytes per thread (D % 16 == 0).
@@ -1160,6 +1219,11 @@ int launch_quantize_mel(const float *mel, float alpha, int8_t *out, int64_t b, i
   return check_launch("quantize_mel_kernel");
 }
 
+// 128 x 128 tiles from here on, where they fill the chip: us with 64 x 64 and 128 x 128
+// tiles, 128 x 1500 x 1280 171 / 148, 64 x 1500 x 1024 63.5 / 50.0, 16 x 1500 x 512 (768 tiles)
+// 8.8 / 6.5, 5 x 1500 x 1024 (480) 6.2 / 5.2, 3 x 677 x 768 (108) 3.1 / 3.5.
+constexpr int64_t kTransposeTiles128 = 400;
+
 int launch_transpose_heads(const int8_t *src, int64_t src_sb, int64_t src_st, int8_t *dst,
                            int64_t dst_sb, int64_t dst_sh, int64_t dst_sd, int64_t dst_sq, int64_t t_off,
                            int64_t B, int64_t T, int64_t H, int64_t D, hipStream_t s) {
@@ -1169,6 +1233,13 @@ int launch_transpose_heads(const int8_t *src, int64_t src_sb, int64_t src_st, in
                        (uintptr_t)src_st | (uintptr_t)dst_sb | (uintptr_t)dst_sh | (uintptr_t)dst_sd |
                        (uintptr_t)t_off | (uintptr_t)(H * D);
   if (dst_sq == 4 && (al & 15) == 0 && H * D <= 0x7fffffff) {
+    const int64_t tt = (T + TH_T - 1) / TH_T, tc = (H * D + TH_C - 1) / TH_C, tiles = tt * tc * B;
+    if (tiles >= kTransposeTiles128 && tiles <= 0x3fffffff) {
+      const unsigned per_xcd = (unsigned)((tiles + 7) / 8);
+      hipLaunchKernelGGL(transpose_heads128_kernel, dim3(8 * per_xcd), dim3(256), 0, s, src, src_sb, src_st, dst, dst_sb,
+                         dst_sh, dst_sd, t_off, T, H, D, (unsigned)tt, (unsigned)tc, (unsigned)tiles, per_xcd);
+      return check_launch("transpose_heads128_kernel");
+    }
     hipLaunchKernelGGL(transpose_heads16_kernel, grid, dim3(256), 0, s, src, src_sb, src_st, dst, dst_sb, dst_sh,
                        dst_sd, t_off, T, H, D);
     return check_launch("transpose_heads16_kernel");
