@@ -24,6 +24,7 @@ _i8 = C.c_int8
 _b = C.c_bool
 _f = C.c_float
 
+
 # name -> argument types (all return int)
 SIGNATURES = {
     "iw_linear8": [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _b, _b, _p],
@@ -35,6 +36,7 @@ SIGNATURES = {
     "iw_add_requant15": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p],
     "iw_conv1d": [_p, _p, _p, _u32, _i8, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _b, _p],
     "iw_classifier": [_p, _p, _u32, _i8, _p, _i64, _i64, _i64, _p],
+    "iw_classifier_dequant": [_p, _p, _u32, _i8, _p, _p, _p, _i64, _i64, _i64, _p],
     "iw_qk_requant_rowmax": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _u8, _i32, _b, _p],
     "iw_shift_exp": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i32, _b, _p],
     "iw_pv_norm_requant": [_p, _p, _p, _u8, _i8, _u32, _p, _i64, _i64, _i64, _i64, _i64, _p],

@@ -43,6 +43,7 @@ struct GemmArgs {
   const int8_t *b = nullptr;
   int64_t ldb = 0;
   int64_t M = 0, N = 0, K = 0;
+  int64_t b_rows = 0;  // rows of b when fewer than N (direct-to-LDS tiles only: the last one is repeated)
   int epi = EPI_L8;
   // epilogue parameters
   const int32_t *bias = nullptr;

@@ -115,6 +115,9 @@ int launch_greedy_update(const uint16_t *amax, int64_t tiles, const int8_t *logi
                          float *sum_logprobs, float scale, int32_t *eot_count, uint32_t *arrive, hipStream_t s);
 int launch_token_prob(const int8_t *logits, int64_t rows, int64_t cols, int64_t ld, int64_t token, float scale,
                       float *out, hipStream_t s);
+// out[m][n] = float(x[m * ld + n]) / *alpha; ld % 16 == 0, x 16-byte aligned
+int launch_dequant_rows(const int8_t *x, int64_t ld, const float *alpha, float *out, int64_t rows, int64_t cols,
+                        hipStream_t s);
 int launch_argmax_rows(const int8_t *x, int64_t rows, int64_t cols, int64_t ld, int64_t *out,
                        hipStream_t s);
 // dst[b*dst_sb + h*dst_sh + d*dst_sd + (t/4)*dst_sq + t%4] for t = t_off + i

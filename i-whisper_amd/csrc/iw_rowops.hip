@@ -902,6 +902,44 @@ __global__ __launch_bounds__(GU_NT) void greedy_update_kernel(GreedyUpdate p) {
   }
 }
 
+// The decoder's float logits: float(x) / alpha of int8 rows with ld bytes between
+// them, written without padding, so that an output row starts at any multiple of 4
+// bytes. A block takes one row's DQ_COLS columns: four floats per thread and
+// store from the row's first 16-byte boundary on (the quad's int8 values come out
+// of two aligned words), and the up to three floats at either end one by one.
+// HBM-bound: 468 x 51865 logits 20 us (as two torch passes 79).
+constexpr int DQ_NT = 256, DQ_COLS = 16 * DQ_NT;
+__global__ __launch_bounds__(DQ_NT) void dequant_rows_kernel(const int8_t *__restrict__ x, int64_t ld,
+                                                             const float *__restrict__ alpha,
+                                                             float *__restrict__ out, int cols) {
+  const int64_t row = blockIdx.y;
+  const int8_t *xr = x + row * ld;
+  float *o = out + row * cols;
+  const float a = *alpha;
+  const int head = min((int)((0 - (reinterpret_cast<uintptr_t>(o) >> 2)) & 3), cols);  // floats before the boundary
+  const int quads = (cols - head) >> 2;
+  const int tail = head + 4 * quads;
+  const uint32_t *xw = reinterpret_cast<const uint32_t *>(xr);
+  const int words = (int)(ld >> 2);
+#pragma unroll
+  for (int i = 0; i < DQ_COLS / (4 * DQ_NT); ++i) {
+    const int q = blockIdx.x * (DQ_COLS / 4) + i * DQ_NT + threadIdx.x;
+    if (q >= quads) continue;
+    // bytes head + 4 q .. + 3; with head = 0 the second word is not used
+    const uint32_t w = __builtin_amdgcn_alignbyte(xw[min(q + 1, words - 1)], xw[q], head);
+    float4 v;
+    v.x = (float)(int8_t)w / a;
+    v.y = (float)(int8_t)(w >> 8) / a;
+    v.z = (float)(int8_t)(w >> 16) / a;
+    v.w = (float)(int8_t)(w >> 24) / a;
+    *reinterpret_cast<float4 *>(o + head + 4 * q) = v;
+  }
+  if (blockIdx.x == 0 && threadIdx.x < 8) {
+    const int c = threadIdx.x < 4 ? (int)threadIdx.x : tail + (int)threadIdx.x - 4;
+    if (threadIdx.x < 4 ? c < head : c < cols) o[c] = (float)xr[c] / a;
+  }
+}
+
 // softmax(logits * scale)[token] of each row in float32 (the no-speech
 // probability at the start-of-transcript position, decoding.py:690-695):
 // exp((x_token - v) * scale) / sum_i exp((x_i - v) * scale), v the row maximum.
@@ -1323,6 +1361,17 @@ int launch_greedy_update(const uint16_t *amax, int64_t tiles, const int8_t *logi
   p.arrive = arrive;
   hipLaunchKernelGGL(greedy_update_kernel, dim3((unsigned)rows), dim3(GU_NT), 0, s, p);
   return check_launch("greedy_update_kernel");
+}
+
+int launch_dequant_rows(const int8_t *x, int64_t ld, const float *alpha, float *out, int64_t rows, int64_t cols,
+                        hipStream_t s) {
+  constexpr int64_t kRowsPerLaunch = 65535;  // grid.y
+  for (int64_t r = 0; r < rows; r += kRowsPerLaunch) {
+    const int64_t n = std::min(rows - r, kRowsPerLaunch);
+    hipLaunchKernelGGL(dequant_rows_kernel, dim3((unsigned)((cols + DQ_COLS - 1) / DQ_COLS), (unsigned)n),
+                       dim3(DQ_NT), 0, s, x + r * ld, ld, alpha, out + r * cols, (int)cols);
+  }
+  return check_launch("dequant_rows_kernel");
 }
 
 int launch_token_prob(const int8_t *logits, int64_t rows, int64_t cols, int64_t ld, int64_t token, float scale,

@@ -336,7 +336,12 @@ class MultiHeadAttention_int(_ScalarCache, nn.Module):
         if mask is not None:  # model_int.py:786-799
             q_offset = Tk - Tq
             assert q_offset >= 0
-            attn_mask = mask[q_offset:q_offset + Tq, :Tk].contiguous()
+            slices = getattr(mask, "attn_slices", None)  # one copy per decoder call, not one per layer
+            attn_mask = None if slices is None else slices.get((Tq, Tk))
+            if attn_mask is None:
+                attn_mask = mask[q_offset:q_offset + Tq, :Tk].contiguous()
+                if slices is not None:
+                    slices[Tq, Tk] = attn_mask
         s = self._scalars()
         out = torch.empty((B, Tq, C), dtype=torch.int8, device=q.device)
         if D % 16 == 0 and D <= 128 and Tk <= 4096:
@@ -606,6 +611,18 @@ class TextDecoder_int(nn.Module):
                   sc["cs"], out.data_ptr(), B * T, C, self.n_vocab, _stream())
         return out
 
+    def _classify_dequant(self, h: Tensor, alpha: Tensor) -> Tensor:
+        """classify(h).float().div(alpha) for a one-element alpha, the division in the same call."""
+        sc = self.scalars()
+        h = h.contiguous()
+        B, T, C = h.shape
+        V = self.n_vocab
+        q8 = torch.empty((B * T, (V + 15) // 16 * 16), dtype=torch.int8, device=h.device)
+        out = torch.empty((B, T, V), dtype=torch.float32, device=h.device)
+        _lib.call("iw_classifier_dequant", h.data_ptr(), self.token_embedding.weight.data_ptr(), sc["cm"],
+                  sc["cs"], alpha.data_ptr(), q8.data_ptr(), out.data_ptr(), B * T, C, V, _stream())
+        return out
+
     def forward(self, x: Tensor, xa: Tensor, kv_cache: Optional[dict] = None):
         check_backend(self.backend)
         offset = next(iter(kv_cache.values())).shape[1] if kv_cache else 0
@@ -614,12 +631,18 @@ class TextDecoder_int(nn.Module):
             if lo < 0 or hi >= self.n_vocab:
                 raise RuntimeError("token id out of range")
         x = self.embed(x, offset)
+        # a view of its own, which carries the slice that the layers of this call share
+        mask = self.mask.view(self.mask.shape)
+        mask.attn_slices = {}
         for block in self.blocks:
-            x = block(x, xa, mask=self.mask, kv_cache=kv_cache)
-        logits = self.classify(self.ln.normalize(x))
-        if self.dequant_need:
-            return logits.float().div(self.act_logits_alpha.detach())
-        return logits
+            x = block(x, xa, mask=mask, kv_cache=kv_cache)
+        h = self.ln.normalize(x)
+        alpha = self.act_logits_alpha.detach()
+        if not self.dequant_need:
+            return self.classify(h)
+        if alpha.numel() == 1 and alpha.dim() <= 3 and alpha.dtype == torch.float32 and alpha.device == h.device:
+            return self._classify_dequant(h, alpha)
+        return self.classify(h).float().div(alpha)
 
     @staticmethod
     def copy_param(quant_layer):

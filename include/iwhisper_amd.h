@@ -119,6 +119,14 @@ int iw_conv1d(const int8_t *x, const int8_t *weight, const int32_t *bias, uint32
 int iw_classifier(const int8_t *x, const int8_t *weight, uint32_t multiplier, int8_t shift,
                   int8_t *out, int64_t M, int64_t K, int64_t N, iw_stream_t stream);
 
+/* The dequantised logits, out[m][n] = float(iw_classifier's int8 logit) / *alpha (alpha a
+ * device float; IEEE division), fp32 [M, N] contiguous: what TextDecoder_int.forward
+ * returns (model_int.py:1446-1490). scratch: M rows of N rounded up to a multiple of
+ * 16 bytes, 16-byte aligned, for the int8 logits. */
+int iw_classifier_dequant(const int8_t *x, const int8_t *weight, uint32_t multiplier, int8_t shift,
+                          const float *alpha, int8_t *scratch, float *out, int64_t M, int64_t K, int64_t N,
+                          iw_stream_t stream);
+
 /* q [B,H,Tq,D], k [B,H,Tk,D] int8; mask [Tq,Tk] or NULL -> qk [B,H,Tq,Tk] int16,
  * row_max_plus1 [B,H,Tq] int16. Replaces iwhisper::qk_requant_rowmax_simd
  * (attention/attention.h:33-46) behind _C.qk_requant_rowmax_simd

@@ -177,6 +177,28 @@ def test_conv1d_channels_last_fused(iw, oracle, gpu, B, Cin, Tin, Cout, stride):
     assert np.array_equal(host(out16), exp16)
 
 
+@pytest.mark.parametrize("M,K,N", [(1, 384, 51865), (5, 40, 33), (3, 64, 1), (128, 128, 1000), (129, 384, 51865),
+                                   (300, 128, 4097), (131, 96, 47), (260, 4096, 35)])
+def test_classifier_dequant(iw, oracle, gpu, M, K, N):
+    """The float logits in one call: rows of N floats at any alignment, the decode
+    kernel and the tiles (whose last 16 columns reach past the weight's rows)."""
+    _print_case("classifier_dequant", M, K, N)
+    r = gen.rng(M + K + N)
+    x, w = gen.i8(r, (1, M, K)), gen.i8(r, (N, K))
+    mult, shift, alpha = 2**30 + 12345, int(np.ceil(np.log2(np.sqrt(K)))) + 4, np.float32(5.83)
+    ld = (N + 15) // 16 * 16
+    q = torch.empty((M, ld), dtype=torch.int8, device="cuda")
+    buf = torch.full((M * N + 8,), -1.0, device="cuda")
+    for off in (0, 3):
+        xt, wt, at = T(x), T(w), torch.tensor([alpha], device="cuda")
+        iw._lib.call("iw_classifier_dequant", xt.data_ptr(), wt.data_ptr(), mult, shift, at.data_ptr(), q.data_ptr(),
+                     buf[off:].data_ptr(), M, K, N, torch.cuda.current_stream().cuda_stream)
+        exp = oracle.classifier(x, w, mult, shift).reshape(-1).astype(np.float32) / alpha
+        assert np.array_equal(host(buf)[off:off + M * N], exp)
+        assert np.all(host(buf)[off + M * N:] == -1.0)
+        buf.fill_(-1.0)
+
+
 # ---------------------------------------------------------------------------
 # Row / element ops
 # ---------------------------------------------------------------------------
