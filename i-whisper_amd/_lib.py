@@ -25,6 +25,14 @@ _b = C.c_bool
 _f = C.c_float
 
 
+class LnInput(C.Structure):
+    """iw_ln_input: the LayerNorm that a decode GEMM computes for its rows."""
+    _fields_ = [("x", _p), ("weight", _p), ("bias", _p), ("out_multiplier", _u32), ("rsqrt_offset", _u32),
+                ("ln_multiplier", _u8), ("ln_shift", _i8), ("out_shift", _i8)]
+
+
+_lnp = C.POINTER(LnInput)
+
 # name -> argument types (all return int)
 SIGNATURES = {
     "iw_linear8": [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _b, _b, _p],
@@ -78,6 +86,11 @@ SIGNATURES = {
     "iw_linear32_residual15_frag": [_p, _p, _p, _p, _p, _p, _p, _u16, _p, _i64, _i64, _i64, _b, _b, _p],
     "iw_linear8_qkv_cache_frag": [_p, _p, _p, _p, _p, _p, _i64, _i64, _b, _b, _p, _i64, _p, _i64, _i64,
                                   _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p],
+    "iw_ln_linear8_frag": [_lnp, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _b, _b, _p],
+    "iw_ln_linear8_gelu_frag": [_lnp, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _i64, _i64,
+                                _i64, _b, _b, _b, _p, _i64, _i64, _p],
+    "iw_ln_linear8_qkv_cache_frag": [_lnp, _p, _p, _p, _p, _p, _i64, _i64, _b, _b, _p, _i64, _p, _i64, _i64,
+                                     _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p],
     "iw_layernorm32_frag": [_p, _p, _p, _u8, _i8, _u32, _i8, _u32, _p, _i64, _i64, _b, _p, _i64, _i64,
                             _p],
     "iw_attention_decode_cross_lnq": [_p, _i64, _p, _p, _u8, _i8, _u32, _i8, _u32, _b, _p, _p, _p, _p, _p, _b, _b,

@@ -904,7 +904,30 @@ int iw_linear8_frag(const int8_t *x, const int8_t *weight, const int32_t *bias, 
   return gemm_frag(g, nullptr, out_frag, as_stream(stream));
 }
 
-int iw_linear8_gelu_frag(const int8_t *x, const int8_t *weight, const int32_t *bias, const int8_t *weight_zero,
+namespace {
+
+// The LayerNorm of a decode GEMM's rows (see LnRows).
+int ln_rows(const iw_ln_input *ln, int64_t M, int64_t K, LnRows *out) {
+  IW_REQUIRE(ln, "null LayerNorm input");
+  IW_REQUIRE(M <= kLnGemmMaxRows, "a decode GEMM with its LayerNorm takes at most 8 rows");
+  IW_REQUIRE(layernorm_width_code(K) >= 0, "unsupported LayerNorm hidden size: " + std::to_string(K));
+  IW_REQUIRE(ln->x && ln->weight, "null LayerNorm pointer");
+  IW_REQUIRE((reinterpret_cast<uintptr_t>(ln->x) & 7) == 0 && (reinterpret_cast<uintptr_t>(ln->weight) & 3) == 0 &&
+                 (reinterpret_cast<uintptr_t>(ln->bias) & 15) == 0,
+             "the LayerNorm's rows must be 8-byte, its weight 4-byte and its bias 16-byte aligned");
+  out->x = ln->x;
+  out->gamma = ln->weight;
+  out->beta = ln->bias;
+  out->ln_m = ln->ln_multiplier;
+  out->ln_s = ln->ln_shift;
+  out->out_m = ln->out_multiplier;
+  out->out_s = ln->out_shift;
+  out->rsqrt_off = ln->rsqrt_offset;
+  out->code = layernorm_width_code(K);
+  return IW_OK;
+}
+
+int linear8_gelu_frag_entry(const int8_t *x, const LnRows &ln, const int8_t *weight, const int32_t *bias, const int8_t *weight_zero,
                          const uint32_t *multiplier, const int8_t *shift, const uint8_t *lut,
                          const uint8_t *luti_multiplier, const int8_t *luti_shift, const uint8_t *luto_multiplier,
                          const int8_t *luto_shift, int64_t luti_count, int64_t luto_count, int8_t *out, int64_t M,
@@ -914,7 +937,7 @@ int iw_linear8_gelu_frag(const int8_t *x, const int8_t *weight, const int32_t *b
   if (rc) return rc;
   rc = check_gelu_counts(N, luti_count, luto_count);
   if (rc || M == 0) return rc;
-  rc = check_frag(x, weight, M, K, N);
+  rc = check_frag(ln.x ? weight : x, weight, M, K, N);
   if (rc) return rc;
   FragPrefetch pf;
   rc = frag_prefetch_args(next_weight, next_n, next_k, &pf);
@@ -923,6 +946,7 @@ int iw_linear8_gelu_frag(const int8_t *x, const int8_t *weight, const int32_t *b
   IW_REQUIRE(lut && luti_multiplier && luti_shift && luto_multiplier && luto_shift, "null GeLU parameter pointer");
   GemmArgs g = linear_args(x, weight, bias, weight_zero, multiplier, shift, out, M, K, N, has_bias, asymmetric,
                            EPI_L8);
+  g.ln = ln;
   g.lut = lut;
   g.luti_m = luti_multiplier;
   g.luti_s = luti_shift;
@@ -933,6 +957,68 @@ int iw_linear8_gelu_frag(const int8_t *x, const int8_t *weight, const int32_t *b
   g.pf = pf;
   if (out_frag) g.ldc = frag_kpad(N);
   return gemm_frag(g, nullptr, out_frag, as_stream(stream));
+}
+
+int linear8_qkv_cache_frag_entry(const int8_t *x, const LnRows &ln, const int8_t *weight, const int32_t *bias,
+                              const int8_t *weight_zero, const uint32_t *multiplier, const int8_t *shift,
+                              int64_t M, int64_t K, bool has_bias, bool asymmetric, int8_t *q_out, int64_t q_ld,
+                              int8_t *k_cache, int64_t k_sb, int64_t k_sh, int64_t k_st, int8_t *v_cache,
+                              int64_t v_sb, int64_t v_sh, int64_t v_sd, int64_t v_sq, int64_t channels,
+                              int64_t head_dim, int64_t tokens_per_row_group, int64_t cache_positions,
+                              const int32_t *pos, iw_stream_t stream) {
+  GemmArgs g;
+  SkinnyScatter sc;
+  int rc = qkv_cache_args(x, weight, bias, weight_zero, multiplier, shift, M, K, has_bias, asymmetric, q_out,
+                          q_ld, k_cache, k_sb, k_sh, k_st, v_cache, v_sb, v_sh, v_sd, v_sq, channels, head_dim,
+                          tokens_per_row_group, cache_positions, pos, &g, &sc);
+  if (rc || M == 0) return rc;
+  rc = check_frag(ln.x ? weight : x, weight, M, K, 3 * channels);
+  if (rc) return rc;
+  g.ln = ln;
+  return gemm_frag(g, &sc, false, as_stream(stream));
+}
+
+}  // namespace
+
+int iw_linear8_gelu_frag(const int8_t *x, const int8_t *weight, const int32_t *bias, const int8_t *weight_zero,
+                         const uint32_t *multiplier, const int8_t *shift, const uint8_t *lut,
+                         const uint8_t *luti_multiplier, const int8_t *luti_shift, const uint8_t *luto_multiplier,
+                         const int8_t *luto_shift, int64_t luti_count, int64_t luto_count, int8_t *out, int64_t M,
+                         int64_t K, int64_t N, bool has_bias, bool asymmetric, bool out_frag,
+                         const int8_t *next_weight, int64_t next_n, int64_t next_k, iw_stream_t stream) {
+  return linear8_gelu_frag_entry(x, LnRows(), weight, bias, weight_zero, multiplier, shift, lut, luti_multiplier,
+      luti_shift, luto_multiplier, luto_shift, luti_count, luto_count, out, M, K, N, has_bias, asymmetric, out_frag,
+      next_weight, next_n, next_k, stream);
+}
+
+int iw_ln_linear8_frag(const iw_ln_input *ln, const int8_t *weight, const int32_t *bias, const int8_t *weight_zero,
+                       const uint32_t *multiplier, const int8_t *shift, int8_t *out, int64_t M, int64_t K, int64_t N,
+                       bool has_bias, bool asymmetric, iw_stream_t stream) {
+  LnRows rows;
+  int rc = ln_rows(ln, M, K, &rows);
+  if (rc) return rc;
+  rc = check_linear(rows.x, weight, bias, weight_zero, multiplier, shift, out, M, K, N, has_bias, asymmetric);
+  if (rc || M == 0) return rc;
+  rc = check_frag(weight, weight, M, K, N);
+  if (rc) return rc;
+  GemmArgs g = linear_args(nullptr, weight, bias, weight_zero, multiplier, shift, out, M, K, N, has_bias, asymmetric,
+                           EPI_L8);
+  g.ln = rows;
+  return gemm_frag(g, nullptr, false, as_stream(stream));
+}
+
+int iw_ln_linear8_gelu_frag(const iw_ln_input *ln, const int8_t *weight, const int32_t *bias, const int8_t *weight_zero,
+                         const uint32_t *multiplier, const int8_t *shift, const uint8_t *lut,
+                         const uint8_t *luti_multiplier, const int8_t *luti_shift, const uint8_t *luto_multiplier,
+                         const int8_t *luto_shift, int64_t luti_count, int64_t luto_count, int8_t *out, int64_t M,
+                         int64_t K, int64_t N, bool has_bias, bool asymmetric, bool out_frag,
+                         const int8_t *next_weight, int64_t next_n, int64_t next_k, iw_stream_t stream) {
+  LnRows rows;
+  const int rc = ln_rows(ln, M, K, &rows);
+  if (rc) return rc;
+  return linear8_gelu_frag_entry(reinterpret_cast<const int8_t *>(rows.x), rows, weight, bias, weight_zero,
+      multiplier, shift, lut, luti_multiplier, luti_shift, luto_multiplier, luto_shift, luti_count, luto_count, out,
+      M, K, N, has_bias, asymmetric, out_frag, next_weight, next_n, next_k, stream);
 }
 
 int iw_linear32_residual15_frag(const int8_t *x, const int8_t *weight, const int32_t *bias,
@@ -959,15 +1045,24 @@ int iw_linear8_qkv_cache_frag(const int8_t *x, const int8_t *weight, const int32
                               int64_t v_sb, int64_t v_sh, int64_t v_sd, int64_t v_sq, int64_t channels,
                               int64_t head_dim, int64_t tokens_per_row_group, int64_t cache_positions,
                               const int32_t *pos, iw_stream_t stream) {
-  GemmArgs g;
-  SkinnyScatter sc;
-  int rc = qkv_cache_args(x, weight, bias, weight_zero, multiplier, shift, M, K, has_bias, asymmetric, q_out,
-                          q_ld, k_cache, k_sb, k_sh, k_st, v_cache, v_sb, v_sh, v_sd, v_sq, channels, head_dim,
-                          tokens_per_row_group, cache_positions, pos, &g, &sc);
-  if (rc || M == 0) return rc;
-  rc = check_frag(x, weight, M, K, 3 * channels);
+  return linear8_qkv_cache_frag_entry(x, LnRows(), weight, bias, weight_zero, multiplier, shift, M, K, has_bias,
+      asymmetric, q_out, q_ld, k_cache, k_sb, k_sh, k_st, v_cache, v_sb, v_sh, v_sd, v_sq, channels, head_dim,
+      tokens_per_row_group, cache_positions, pos, stream);
+}
+
+int iw_ln_linear8_qkv_cache_frag(const iw_ln_input *ln, const int8_t *weight, const int32_t *bias,
+                              const int8_t *weight_zero, const uint32_t *multiplier, const int8_t *shift,
+                              int64_t M, int64_t K, bool has_bias, bool asymmetric, int8_t *q_out, int64_t q_ld,
+                              int8_t *k_cache, int64_t k_sb, int64_t k_sh, int64_t k_st, int8_t *v_cache,
+                              int64_t v_sb, int64_t v_sh, int64_t v_sd, int64_t v_sq, int64_t channels,
+                              int64_t head_dim, int64_t tokens_per_row_group, int64_t cache_positions,
+                              const int32_t *pos, iw_stream_t stream) {
+  LnRows rows;
+  const int rc = ln_rows(ln, M, K, &rows);
   if (rc) return rc;
-  return gemm_frag(g, &sc, false, as_stream(stream));
+  return linear8_qkv_cache_frag_entry(reinterpret_cast<const int8_t *>(rows.x), rows, weight, bias, weight_zero,
+      multiplier, shift, M, K, has_bias, asymmetric, q_out, q_ld, k_cache, k_sb, k_sh, k_st, v_cache, v_sb, v_sh,
+      v_sd, v_sq, channels, head_dim, tokens_per_row_group, cache_positions, pos, stream);
 }
 
 int iw_layernorm32_frag(const int16_t *x, const int8_t *weight, const int32_t *bias, uint8_t ln_multiplier,

@@ -33,6 +33,22 @@ struct FragPrefetch {
   int blocks = 0, threads = 0;
 };
 
+// The LayerNorm32 of residual rows that a decode GEMM computes itself (gemm_frag
+// with g.ln.x set): x is [M][K] int16, beta may be null; gamma is 4-byte, beta
+// 16-byte aligned.
+struct LnRows {
+  const int16_t *x = nullptr;
+  const int8_t *gamma = nullptr;
+  const int32_t *beta = nullptr;
+  uint32_t ln_m = 0;
+  int32_t ln_s = 0;
+  uint32_t out_m = 0;
+  int32_t out_s = 0;
+  uint32_t rsqrt_off = 0;
+  int32_t code = 0;  // layernorm_width_code(K)
+};
+constexpr int64_t kLnGemmMaxRows = 8;
+
 struct GemmArgs {
   // A operand
   const int8_t *a = nullptr;
@@ -74,6 +90,7 @@ struct GemmArgs {
   void *out = nullptr;
   int64_t ldc = 0;
   int64_t out_T = 1;  // OUT_NCT: rows are (b, t) with t in [0, out_T)
+  LnRows ln;  // gemm_frag only: a is not used
   // the next decode GEMM's weight, read into L2 (gemm_frag_kernel only)
   FragPrefetch pf;
   // per-tensor int8 epilogue (classifier) only, gemm_frag_kernel: the first

@@ -53,10 +53,98 @@ __device__ __forceinline__ void classifier_argmax_store(const GemmArgs &g, const
   if ((lane & 31) == 0 && m < (int)g.M) g.amax[(int64_t)m * g.amax_ld + tile] = (uint16_t)k;
 }
 
+// LayerNorm32 of one row by one wave, lane l taking the 4-element chunks l, l + 64,
+// ... (the integer steps of layernorm32_row_kernel), in two parts so that other
+// loads can follow the row's own.
+struct LnChunks {
+  static constexpr int N = 5;  // 1280 / 4 / 64
+  uint2 x[N];
+  uint32_t g[N];
+  uint4 b[N];
+};
+
+__device__ __forceinline__ void ln_wave_load(const LnRows &ln, int64_t row, int hidden, LnChunks &r) {
+  const int lane = threadIdx.x & 63, nch = hidden >> 2;
+  const int16_t *xr = ln.x + row * hidden;
+#pragma unroll
+  for (int c = 0; c < LnChunks::N; ++c) {
+    const int ch = lane + 64 * c;
+    r.x[c] = make_uint2(0, 0);
+    r.g[c] = 0;
+    r.b[c] = make_uint4(0, 0, 0, 0);
+    if (ch < nch) {
+      r.x[c] = *reinterpret_cast<const uint2 *>(xr + ch * 4);
+      r.g[c] = *reinterpret_cast<const uint32_t *>(ln.gamma + ch * 4);
+      if (ln.beta) r.b[c] = *reinterpret_cast<const uint4 *>(ln.beta + ch * 4);
+    }
+  }
+}
+
+// dst: the row's kp bytes in LDS, zeros past hidden
+__device__ __forceinline__ void ln_wave_row(const LnRows &ln, const LnChunks &r, int hidden, int kp, int8_t *dst) {
+  const int lane = threadIdx.x & 63, nch = hidden >> 2;
+  int32_t d[LnChunks::N][4];
+  uint32_t sum = 0;
+#pragma unroll
+  for (int c = 0; c < LnChunks::N; ++c) {
+    d[c][0] = (int16_t)(r.x[c].x & 0xffff), d[c][1] = (int16_t)(r.x[c].x >> 16);
+    d[c][2] = (int16_t)(r.x[c].y & 0xffff), d[c][3] = (int16_t)(r.x[c].y >> 16);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum += (uint32_t)d[c][e];  // zeros past the row
+  }
+  const int32_t mean = norm_reduce((int32_t)wave_sum_dpp(sum), ln.code);
+  int32_t maxsq = 0;
+#pragma unroll
+  for (int c = 0; c < LnChunks::N; ++c)
+    if (lane + 64 * c < nch)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        d[c][e] -= mean;
+        maxsq = max(maxsq, (int32_t)((uint32_t)d[c][e] * (uint32_t)d[c][e]));
+      }
+  maxsq = wave_max_dpp(maxsq);
+  int32_t rs = bitlen(maxsq) - 16;
+  rs = rs < 0 ? 0 : rs;
+  rs = (rs + 1) & ~1;
+  uint32_t vs = 0;
+#pragma unroll
+  for (int c = 0; c < LnChunks::N; ++c)
+    if (lane + 64 * c < nch)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vs += (uint32_t)rshift((int32_t)((uint32_t)d[c][e] * (uint32_t)d[c][e]), (uint32_t)rs);
+  const int32_t inv = fisr(norm_reduce((int32_t)wave_sum_dpp(vs), ln.code), ln.rsqrt_off);
+  const uint32_t nshift = (uint32_t)(ln.ln_s + (rs >> 1));
+#pragma unroll
+  for (int c = 0; c < LnChunks::N; ++c) {
+    const int ch = lane + 64 * c;
+    if (ch < nch) {
+      const uint32_t bv[4] = {r.b[c].x, r.b[c].y, r.b[c].z, r.b[c].w};
+      uint32_t packed = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t t = (uint32_t)d[c][e] * (uint32_t)inv * ln.ln_m;
+        const int32_t y = clampi(rshift((int32_t)t, nshift), -16383, 16383);
+        const uint32_t a = (uint32_t)y * (uint32_t)(int32_t)(int8_t)(r.g[c] >> (8 * e)) + bv[e];
+        const int32_t o = clampi(rshift(mulh((int32_t)a, ln.out_m), (uint32_t)ln.out_s), -127, 127);
+        packed |= (uint32_t)(uint8_t)(int8_t)o << (8 * e);
+      }
+      *reinterpret_cast<uint32_t *>(dst + ch * 4) = packed;
+    }
+  }
+  for (int k = hidden + lane * 4; k < kp; k += 256) *reinterpret_cast<uint32_t *>(dst + k) = 0;
+}
+
 // Each wave multiplies the block's 32 x 32 tile over SPW k32 steps; a block
 // has MINW .. MAXW waves (MINW bounds the epilogue rows a thread serves).
 // ARGMAX: the classifier epilogue that also writes the per-tile row maxima.
-template <int EPI, bool GELU, bool SCATTER, bool OUT_FRAG, int SPW, int MAXW, int MINW, bool ARGMAX = false>
+// LN: A is the LayerNorm of g.ln's rows (at most kLnGemmMaxRows), which every block
+// computes for itself, a wave a row, while its weights are on the way: the launch
+// bound steps of a few rows lose a launch per LayerNorm. us per token step with and
+// without: one row of tiny / base / small / medium / large 226 / 244, 258 / 274, 518 / 554,
+// 1183 / 1290, 1684 / 1808; five rows (a second row for some waves) 249 / 251, 279 / 282,
+// 594 / 632, 1242 / 1290, 1768 / 1820; eight 253 / 253, 283 / 286, 627 / 638, 1250 / 1302, 1771 / 1829.
+template <int EPI, bool GELU, bool SCATTER, bool OUT_FRAG, int SPW, int MAXW, int MINW, bool ARGMAX = false,
+          bool LN = false>
 __global__ __launch_bounds__(64 * MAXW) void gemm_frag_kernel(GemmArgs g, SkinnyScatter sc, int ms, int tiles,
                                                               int kp) {
   // the waves' partial tiles are added into one tile in LDS (ds_add); row
@@ -66,6 +154,8 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_frag_kernel(GemmArgs g, Skinny
   __shared__ int32_t sTile[32 * PLD];
   __shared__ int32_t sXs[32];
   __shared__ uint8_t sLut[16];
+  constexpr int LDH = LN ? 32 * SPW * MAXW + 16 : 16;  // LayerNorm rows in LDS
+  __shared__ __attribute__((aligned(16))) int8_t sH[LN ? kLnGemmMaxRows * LDH : 16];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -76,6 +166,13 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_frag_kernel(GemmArgs g, Skinny
   if (tile >= tiles) return;
   const int M = (int)g.M, N = (int)g.N;
   const int m0 = msub * 32, n0 = tile * 32;
+
+  // the rows to normalise before all else: the chain starts with them
+  LnChunks lr;
+  if constexpr (LN) {
+    ln_wave_load(g.ln, min(wave, M - 1), (int)g.K, lr);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   // epilogue inputs first: in a decode step they are as cold as the weights
   // (per-layer parameters, the residual rows just written), and requested
@@ -109,7 +206,7 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_frag_kernel(GemmArgs g, Skinny
   v4i fa[SPW], fb[SPW];
 #pragma unroll
   for (int t = 0; t < SPW; ++t) {
-    fa[t] = *reinterpret_cast<const v4i *>(pa + t * 1024);
+    if (!LN) fa[t] = *reinterpret_cast<const v4i *>(pa + t * 1024);
     fb[t] = *reinterpret_cast<const v4i *>(pb + t * 1024);
   }
   // FC1 (the GeLU instances) reads FC2's weight tiles into L2 behind its own
@@ -126,11 +223,28 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_frag_kernel(GemmArgs g, Skinny
     __builtin_amdgcn_sched_barrier(0);
   }
 
+  if constexpr (LN) {
+    __builtin_amdgcn_sched_barrier(0);
+    for (int r = wave; r < M; r += nt >> 6) {
+      if (r != wave) ln_wave_load(g.ln, r, (int)g.K, lr);
+      ln_wave_row(g.ln, lr, (int)g.K, kp, &sH[r * LDH]);
+    }
+  }
+
   // the zeroed tile is seen by every wave before any adds into it (an LDS-only
   // barrier: the operand loads stay in flight)
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
+
+  if constexpr (LN) {
+    const int r = lane & 31;
+#pragma unroll
+    for (int t = 0; t < SPW; ++t) {
+      fa[t] = v4i{0, 0, 0, 0};
+      if (r < M) fa[t] = *reinterpret_cast<const v4i *>(&sH[r * LDH + (wave * SPW + t) * 32 + (lane >> 5) * 16]);
+    }
+  }
 
   // two accumulator chains so that consecutive MFMAs do not wait on each
   // other; row sums of A for the zero-point term from the same registers
@@ -189,7 +303,8 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_frag_kernel(GemmArgs g, Skinny
   if constexpr (PF) frag_prefetch_keep(pfv);
 }
 
-template <int EPI, bool GELU, bool SCATTER, bool OUT_FRAG, int SPW, int MAXW, int MINW, bool ARGMAX = false>
+template <int EPI, bool GELU, bool SCATTER, bool OUT_FRAG, int SPW, int MAXW, int MINW, bool ARGMAX = false,
+          bool LN = false>
 int launch_frag_waves(const GemmArgs &g, const SkinnyScatter &sc, int64_t kp, hipStream_t s) {
   const int64_t tiles = (g.N + 31) / 32;
   const int ms = (int)((g.M + 31) / 32);
@@ -197,8 +312,8 @@ int launch_frag_waves(const GemmArgs &g, const SkinnyScatter &sc, int64_t kp, hi
   const dim3 grid((unsigned)(((tiles + 7) / 8) * 8 * ms));
   GemmArgs ga = g;
   frag_prefetch_launch(ga.pf, grid.x, 64 * nw);
-  hipLaunchKernelGGL((gemm_frag_kernel<EPI, GELU, SCATTER, OUT_FRAG, SPW, MAXW, MINW, ARGMAX>), grid, dim3(64 * nw),
-                     0, s, ga, sc, ms, (int)tiles, (int)kp);
+  hipLaunchKernelGGL((gemm_frag_kernel<EPI, GELU, SCATTER, OUT_FRAG, SPW, MAXW, MINW, ARGMAX, LN>), grid,
+                     dim3(64 * nw), 0, s, ga, sc, ms, (int)tiles, (int)kp);
   return check_launch("gemm_frag_kernel");
 }
 
@@ -209,6 +324,9 @@ int launch_frag_waves(const GemmArgs &g, const SkinnyScatter &sc, int64_t kp, hi
 template <int EPI, bool GELU, bool SCATTER, bool OUT_FRAG, bool ARGMAX = false>
 int launch_frag(const GemmArgs &g, const SkinnyScatter &sc, hipStream_t s) {
   const int64_t kp = frag_kpad(g.K);
+  if constexpr (EPI == EPI_L8 && !ARGMAX && GELU == OUT_FRAG) {
+    if (g.ln.x) return launch_frag_waves<EPI, GELU, SCATTER, OUT_FRAG, 5, 8, 2, false, true>(g, sc, kp, s);
+  }
   if (kp <= 1280) return launch_frag_waves<EPI, GELU, SCATTER, OUT_FRAG, 5, 8, 2, ARGMAX>(g, sc, kp, s);
   if (kp <= 2560) return launch_frag_waves<EPI, GELU, SCATTER, OUT_FRAG, 10, 8, 5, ARGMAX>(g, sc, kp, s);
   return launch_frag_waves<EPI, GELU, SCATTER, OUT_FRAG, 10, 16, 9, ARGMAX>(g, sc, kp, s);
@@ -246,6 +364,8 @@ __global__ __launch_bounds__(256) void frag_pack_kernel(const int8_t *__restrict
 int gemm_frag(const GemmArgs &g, const SkinnyScatter *scatter, bool out_frag, hipStream_t s) {
   if (g.M == 0) return 0;
   const bool gelu = g.lut != nullptr;
+  if (g.ln.x && (g.M > kLnGemmMaxRows || g.epi != EPI_L8 || gelu != out_frag || frag_kpad(g.K) > 1280))
+    return fail("the GEMM with its LayerNorm takes 8 rows, 1280 columns and Linear8");
   SkinnyScatter sc;
   if (scatter) {
     if (g.epi != EPI_L8 || gelu || out_frag) return fail("the KV-cache epilogue is for the Linear8 QKV projection");

@@ -152,6 +152,22 @@ def _ln_frag(ln, x: torch.Tensor, rows: int, out: torch.Tensor, nxt: Optional["_
     return out
 
 
+# Rows up to which the decode GEMMs of a token step compute their LayerNorm
+# themselves (see iw_gemm_frag.hip).
+LN_GEMM_ROWS = 8
+
+
+def _ln_gemm_ok(ln) -> bool:
+    """Whether the decode GEMMs can read this LayerNorm's parameters (whole words)."""
+    return ln.weight.data_ptr() % 4 == 0 and (ln.bias is None or ln.bias.data_ptr() % 16 == 0)
+
+
+def _ln_input(ln, x: torch.Tensor):
+    s = ln._scalars()
+    return _lib.LnInput(x.data_ptr(), ln.weight.data_ptr(), _ptr(ln.bias), s["om"], ln.offset, s["lm"], s["ls"],
+                        s["os"])
+
+
 class _FragLinear:
     """A LinearBase layer (or a _FusedLinear) with its weight packed
     fragment-major for the one-token decode GEMMs."""
@@ -363,6 +379,8 @@ class DecoderRunner:
         # GEMM's weight tiles into L2 (a hint; results do not depend on it)
         self.prefetch = prefetch
         self.fuse_cross = fuse_cross and self.frag and self.D == 64 and n_audio_ctx <= 2048
+        self.ln_gemm = self.frag and batch <= LN_GEMM_ROWS and C <= 1280 and all(
+            _ln_gemm_ok(n) for b in decoder.blocks for n in (b.attn_ln, b.cross_attn_ln, b.mlp_ln))
         if self.frag:
             self.f_qkv = [_FragLinear(f) for f in self.self_qkv]
             self.f_out = [_FragLinear(b.attn.out) for b in decoder.blocks]
@@ -643,8 +661,12 @@ class DecoderRunner:
         for l, blk in enumerate(dec.blocks):
             sc = blk._scalars()
             fq = self.f_qkv[l]
-            _ln_frag(blk.attn_ln, x16, B, h8f, pf(fq))
-            _lib.call("iw_linear8_qkv_cache_frag", h8f.data_ptr(), *fq.args(), B, C, True, True,
+            if self.ln_gemm:
+                entry, h_in = "iw_ln_linear8_qkv_cache_frag", _ln_input(blk.attn_ln, x16)
+            else:
+                entry, h_in = "iw_linear8_qkv_cache_frag", h8f.data_ptr()
+                _ln_frag(blk.attn_ln, x16, B, h8f, pf(fq))
+            _lib.call(entry, h_in, *fq.args(), B, C, True, True,
                       q8.data_ptr(), C, self.k_self[l].data_ptr(), H * self.Tcap * D, self.Tcap * D, D,
                       self.v_self[l].data_ptr(), *self.v_strides, C, D, 1, self.Tcap, self.pos.data_ptr(),
                       _stream())
@@ -660,18 +682,27 @@ class DecoderRunner:
             if self.fuse_cross:
                 self._cross_lnq(l, wvf)
             else:
-                _ln_frag(blk.cross_attn_ln, x16, B, h8f, pf(self.f_cq[l]))
-                self.f_cq[l].linear8(h8f, B, q8)
+                cq = self.f_cq[l]
+                if self.ln_gemm:
+                    _lib.call("iw_ln_linear8_frag", _ln_input(blk.cross_attn_ln, x16), *cq.args(), q8.data_ptr(), B,
+                              cq.K, cq.N, cq.bias is not None, cq.wz is not None, _stream())
+                else:
+                    _ln_frag(blk.cross_attn_ln, x16, B, h8f, pf(cq))
+                    cq.linear8(h8f, B, q8)
                 _lib.call("iw_attention_decode_cache_frag", q8.data_ptr(), C, self.k_cross[l].data_ptr(),
                           H * Ta * D, Ta * D, D, self.vt_cross[l].data_ptr(), H * D * self.ta16,
                           D * self.ta16, self.ta16, 4, wvf.data_ptr(), B, H, D, Ta, None, Ta, s["qm"], s["qs"],
                           s["f"], s["am"], s["as_"], blk.cross_attn.rsqrt_offset, *_NO_PREFETCH, _stream())
             self.f_co[l].linear32_res(wvf, B, x16, sc["c"])
             f1, f2 = self.f_fc1[l], self.f_fc2[l]
-            _ln_frag(blk.mlp_ln, x16, B, h8f, pf(f1))
+            if self.ln_gemm:
+                entry, h_in = "iw_ln_linear8_gelu_frag", _ln_input(blk.mlp_ln, x16)
+            else:
+                entry, h_in = "iw_linear8_gelu_frag", h8f.data_ptr()
+                _ln_frag(blk.mlp_ln, x16, B, h8f, pf(f1))
             lut, im, is_, om, os_, ci, co = blk.mlp[1].gelu_ptrs()
             nxt = pf(f2)
-            _lib.call("iw_linear8_gelu_frag", h8f.data_ptr(), *f1.args(), lut, im, is_, om, os_, ci, co,
+            _lib.call(entry, h_in, *f1.args(), lut, im, is_, om, os_, ci, co,
                       f8f.data_ptr(), B, f1.K, f1.N, f1.bias is not None, f1.wz is not None, True,
                       *_pf_args(nxt), _stream())
             f2.linear32_res(f8f, B, x16, sc["m"])

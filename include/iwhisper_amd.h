@@ -429,6 +429,39 @@ int iw_linear8_qkv_cache_frag(const int8_t *x, const int8_t *weight, const int32
                               int64_t channels, int64_t head_dim, int64_t tokens_per_row_group,
                               int64_t cache_positions, const int32_t *pos, iw_stream_t stream);
 
+/* The same three decode GEMMs computing the LayerNorm32 of their input rows themselves
+ * (M <= 8 rows of K = 384, 512, 768, 1024 or 1280 residuals, bit for bit iw_layernorm32_frag
+ * followed by the GEMM): one launch instead of two. bias may be NULL; x is 8-byte, weight
+ * 4-byte and bias 16-byte aligned. The struct is read during the call. */
+typedef struct iw_ln_input {
+  const int16_t *x;
+  const int8_t *weight;
+  const int32_t *bias;
+  uint32_t out_multiplier;
+  uint32_t rsqrt_offset;
+  uint8_t ln_multiplier;
+  int8_t ln_shift;
+  int8_t out_shift;
+} iw_ln_input;
+int iw_ln_linear8_frag(const iw_ln_input *ln, const int8_t *weight, const int32_t *bias, const int8_t *weight_zero,
+                       const uint32_t *multiplier, const int8_t *shift, int8_t *out, int64_t M, int64_t K, int64_t N,
+                       bool has_bias, bool asymmetric, iw_stream_t stream);
+int iw_ln_linear8_gelu_frag(const iw_ln_input *ln, const int8_t *weight, const int32_t *bias,
+                         const int8_t *weight_zero, const uint32_t *multiplier, const int8_t *shift,
+                         const uint8_t *lut, const uint8_t *luti_multiplier, const int8_t *luti_shift,
+                         const uint8_t *luto_multiplier, const int8_t *luto_shift, int64_t luti_count,
+                         int64_t luto_count, int8_t *out, int64_t M, int64_t K, int64_t N,
+                         bool has_bias, bool asymmetric, bool out_frag, const int8_t *next_weight,
+                         int64_t next_n, int64_t next_k, iw_stream_t stream);
+int iw_ln_linear8_qkv_cache_frag(const iw_ln_input *ln, const int8_t *weight, const int32_t *bias,
+                              const int8_t *weight_zero, const uint32_t *multiplier,
+                              const int8_t *shift, int64_t M, int64_t K, bool has_bias,
+                              bool asymmetric, int8_t *q_out, int64_t q_ld, int8_t *k_cache,
+                              int64_t k_sb, int64_t k_sh, int64_t k_st, int8_t *v_cache,
+                              int64_t v_sb, int64_t v_sh, int64_t v_sd, int64_t v_sq,
+                              int64_t channels, int64_t head_dim, int64_t tokens_per_row_group,
+                              int64_t cache_positions, const int32_t *pos, iw_stream_t stream);
+
 /* iw_layernorm32 writing the fragment-major image of out [rows][hidden]
  * (rows <= 128); next_weight / next_n / next_k: the prefetch hint of
  * iw_linear8_gelu_frag (the GEMM that reads out). */

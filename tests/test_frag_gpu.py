@@ -274,6 +274,68 @@ def test_linear8_qkv_cache_frag(iw, oracle, gpu, B, H, D, pos_val, tcap, layout)
     assert np.array_equal(host(vc), vexp)
 
 
+@pytest.mark.parametrize("hidden,rows,spread,beta", [(384, 1, 4000, True), (384, 8, 0, True), (512, 5, 16000, True),
+                                                     (768, 7, 300, False), (1024, 8, 4000, True),
+                                                     (1280, 1, 16000, True), (1280, 8, 30000, True)])
+def test_ln_gemm_frag(iw, oracle, gpu, hidden, rows, spread, beta):
+    """The decode GEMMs that compute their rows' LayerNorm: one row and eight,
+    K padded and not, constant rows and deviations whose squares wrap."""
+    print("case: ln gemm frag", hidden, rows, spread, beta, flush=True)
+    x, g, b, lm, ls, om, os_ = gen.ln_case(hidden + rows, rows, hidden, spread)
+    if spread == 30000:
+        x[0], x[0, 5] = 32767, -32768
+    h = oracle.layernorm32(x, g, b if beta else None, lm, ls, om, os_)
+    xt, gt, bt = T(x), T(g), T(b)
+    ln = iw._lib.LnInput(xt.data_ptr(), gt.data_ptr(), bt.data_ptr() if beta else None, om, 13, lm, ls, os_)
+    # plain Linear8, no bias and symmetric beside both
+    for has_bias, asym in ((True, True), (False, False)):
+        _, w, bias, z, m, s = gen.realistic_linear_case(rows + hidden, rows, hidden, 200)
+        wf, bs, zs, ms, ss = pack(iw, w), T(bias), T(z), T(m), T(s)
+        out = torch.empty((rows, 200), dtype=torch.int8, device="cuda")
+        iw._lib.call("iw_ln_linear8_frag", ln, wf.data_ptr(), bs.data_ptr(), zs.data_ptr(), ms.data_ptr(),
+                     ss.data_ptr(), out.data_ptr(), rows, hidden, 200, has_bias, asym, stream())
+        assert np.array_equal(host(out), oracle.linear8(h, w, bias if has_bias else None, z if asym else None, m, s))
+    # FC1 with GeLU, its output fragment-major
+    N = 4 * hidden
+    _, w, bias, z, m, s = gen.realistic_linear_case(rows + N, rows, hidden, N)
+    r = gen.rng(N)
+    gp = gen.gelu_params(r, N)
+    ts = [T(a) for a in (bias, z, m, s, *gp)]
+    wf, of = pack(iw, w), zeros_frag(iw, rows, N)
+    iw._lib.call("iw_ln_linear8_gelu_frag", ln, wf.data_ptr(), *[t.data_ptr() for t in ts], N, N, of.data_ptr(), rows,
+                 hidden, N, True, True, True, None, 0, 0, stream())
+    assert np.array_equal(host(of), frag_image(oracle.gelu(oracle.linear8(h, w, bias, z, m, s), *gp)))
+    # QKV with the cache append
+    H, D, tcap = hidden // 64, 64, 48
+    _, w, bias, z, m, s = gen.realistic_linear_case(rows + 3, rows, hidden, 3 * hidden)
+    e = oracle.linear8(h, w, bias, z, m, s)
+    kc0, (shape, vs) = gen.i8(r, (rows, H, tcap, D)), gen.v_cache_layout(rows, H, D, tcap, "quads")
+    vc0 = gen.i8(r, shape)
+    kc, vc, q = T(kc0), T(vc0), torch.empty((rows, hidden), dtype=torch.int8, device="cuda")
+    pos = torch.tensor([17], dtype=torch.int32, device="cuda")
+    ts, wf = [T(a) for a in (bias, z, m, s)], pack(iw, w)
+    iw._lib.call("iw_ln_linear8_qkv_cache_frag", ln, wf.data_ptr(), *[t.data_ptr() for t in ts], rows, hidden, True,
+                 True, q.data_ptr(), hidden, kc.data_ptr(), H * tcap * D, tcap * D, D, vc.data_ptr(), *vs, hidden, D,
+                 1, tcap, pos.data_ptr(), stream())
+    assert np.array_equal(host(q), e[:, :hidden])
+    e = e.reshape(rows, 3, H, D)
+    kc0[:, :, 17, :] = e[:, 1]
+    gen.v_cache_put(vc0, "quads", 17, e[:, 2][..., None])
+    assert np.array_equal(host(kc), kc0) and np.array_equal(host(vc), vc0)
+
+
+def test_ln_gemm_frag_rejects(iw, gpu):
+    x = torch.zeros((9, 384), dtype=torch.int16, device="cuda")
+    g = torch.ones(400, dtype=torch.int8, device="cuda")
+    w = torch.zeros(iw._lib.value("iw_frag_bytes", 32, 384), dtype=torch.int8, device="cuda")
+    m = torch.ones(32, dtype=torch.int32, device="cuda")
+    for rows, hidden, goff in ((9, 384, 0), (1, 400, 0), (1, 384, 1)):
+        ln = iw._lib.LnInput(x.data_ptr(), g.data_ptr() + goff, None, 1, 13, 1, 1, 1)
+        with pytest.raises(RuntimeError, match="at most 8 rows|hidden size|aligned"):
+            iw._lib.call("iw_ln_linear8_frag", ln, w.data_ptr(), None, None, m.data_ptr(), g.data_ptr(),
+                         w.data_ptr(), rows, hidden, 32, False, False, stream())
+
+
 def test_frag_gemm_rejects_large_k(iw, gpu):
     x = torch.zeros(iw._lib.value("iw_frag_bytes", 4, 5120), dtype=torch.int8, device="cuda")
     m = torch.ones(8, dtype=torch.int32, device="cuda")
