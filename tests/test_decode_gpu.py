@@ -209,6 +209,13 @@ def test_transpose_heads(iw, gpu, B, T, H, D, t_off, layout):
     assert np.array_equal(host(dst), exp)
 
 
+@pytest.mark.parametrize("B,T,H,D,t_off", [(60, 333, 7, 48, 16), (5, 1500, 16, 64, 0), (200, 130, 2, 64, 0),
+                                           (401, 1, 1, 16, 0)])
+def test_transpose_heads_many(iw, gpu, B, T, H, D, t_off):
+    """Enough 128 x 128 tiles for the large form: ragged positions and columns."""
+    test_transpose_heads(iw, gpu, B, T, H, D, t_off, "vt")
+
+
 def test_embed_tokens(iw, oracle, gpu):
     r = gen.rng(11)
     B, V, C, n_ctx = 6, 500, 128, 40
