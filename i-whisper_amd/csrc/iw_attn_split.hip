@@ -22,7 +22,7 @@ namespace iw {
 namespace {
 
 constexpr int KC = 32;  // keys per chunk
-constexpr int NW = 4;   // waves of a block
+constexpr int kHold = 6, kAhead = 3;  // chunks of a wave whose K it holds, V^T chunks ahead
 
 // Where this kernel runs (tiles of 32 queries; measured against 128 queries
 // per block, us):
@@ -39,11 +39,21 @@ constexpr int NW = 4;   // waves of a block
 //   (376 -> 22.7, 7520 -> 226 against 164).
 // Above kSplitPairTiles (three blocks per CU) a wave takes two tiles over one
 // set of K / V^T fragments: 940 tiles 42.1 -> 35.6, 1504 tiles 55.2 -> 46.9.
-constexpr int64_t kSplitMaxTiles = 1600, kSplitPairTiles = 768;
+// Eight waves that hold their K fragments (HOLD) for 9 .. 48 chunks of keys, us with
+// four waves and with eight: 117 queries of 48 heads over 1500 keys (192 tiles)
+// 15.7 -> 11.7, 8 heads over 1500 positions (376; pairs, one block per CU) 22.5 -> 18.1, 12
+// queries of 320 / 2560 heads 24.5 -> 23.2 / 166 -> 146, 4 heads of 96 (188) 18.9 -> 15.8 and 16
+// (752) 53 -> 43; not at 564 tiles of 64 (30.5 / 31.7), 64 heads of 96 (144 / 161), 117 keys
+// (9.6 / 12.2: the chunks past the last are read for nothing) or head_dim 128 (spills).
+constexpr int64_t kSplitMaxTiles = 1600, kSplitPairTiles = 768, kCus = 256;
 
 // QT: 32-query subtiles per wave, all over the same K and V^T fragments.
-template <int KS, bool HAS_MASK, bool DF, int QT>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(KS <= 2 && QT == 1 ? 4 : 2)))
+// HOLD: at most kHold chunks per wave, whose K fragments are all requested at the
+// start and kept for pass 2, and whose V^T fragments are requested kAhead chunks ahead:
+// two waves per SIMD hide little of a load's latency, which otherwise
+// comes once per chunk and pass.
+template <int KS, bool HAS_MASK, bool DF, int QT, int NW, bool HOLD>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(!HOLD && KS <= 2 && QT == 1 ? 4 : 2)))
 void attn_prefill_split_kernel(AttnArgs a, int qtiles, int tiles, int per_xcd) {
   constexpr int DP = KS * 32, OLD = DP + 1, QR = 32 * QT;
   static_assert(QR * OLD * 4 <= IW_SEXP_LUT, "the output tile fits in the table's space");
@@ -133,6 +143,7 @@ void attn_prefill_split_kernel(AttnArgs a, int qtiles, int tiles, int per_xcd) {
   const int nkc = (Tk + KC - 1) / KC;
   const int nfk = HAS_MASK ? 0 : Tk / KC;  // chunks in which every key counts
   v4i kf[KS], kn[KS];
+  v4i kh[HOLD ? kHold : 1][KS], vh[HOLD ? kAhead : 1][KS];
   auto next_k = [&](int kc) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) kf[ks] = kn[ks];
@@ -143,21 +154,36 @@ void attn_prefill_split_kernel(AttnArgs a, int qtiles, int tiles, int per_xcd) {
   int32_t mx[QT];
 #pragma unroll
   for (int u = 0; u < QT; ++u) mx[u] = INT32_MIN;
-  if (wave < nkc) load_k(wave, kn);
-  for (int kc = wave; kc < nkc; kc += NW) {
-    next_k(kc);
+  auto chunk_max = [&](int kc, const v4i (&f)[KS]) {
 #pragma unroll
-      for (int u = 0; u < QT; ++u) {
-        const v16i s = scores(kf, u);
-        if (kc < nfk) {
+    for (int u = 0; u < QT; ++u) {
+      const v16i s = scores(f, u);
+      if (kc < nfk) {
 #pragma unroll
-          for (int r = 0; r < 16; r += 2) mx[u] = max(max(mx[u], s[r]), s[r + 1]);
-        } else {
+        for (int r = 0; r < 16; r += 2) mx[u] = max(max(mx[u], s[r]), s[r + 1]);
+      } else {
 #pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (counts(u, kc * KC + g * 16 + r)) mx[u] = max(mx[u], s[r]);
-        }
+        for (int r = 0; r < 16; ++r)
+          if (counts(u, kc * KC + g * 16 + r)) mx[u] = max(mx[u], s[r]);
       }
+    }
+  };
+  if constexpr (HOLD) {
+    // chunks past the last read it again and are not used
+#pragma unroll
+    for (int i = 0; i < kHold; ++i) load_k(min(wave + NW * i, nkc - 1), kh[i]);
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) load_v(min(wave + NW * i, nkc - 1), vh[i]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kHold; ++i)
+      if (wave + NW * i < nkc) chunk_max(wave + NW * i, kh[i]);
+  } else {
+    if (wave < nkc) load_k(wave, kn);
+    for (int kc = wave; kc < nkc; kc += NW) {
+      next_k(kc);
+      chunk_max(kc, kf);
+    }
   }
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
@@ -165,7 +191,7 @@ void attn_prefill_split_kernel(AttnArgs a, int qtiles, int tiles, int per_xcd) {
     if (lane < 32) sMax[wave][32 * u + lane] = mx[u];
   }
   if (tid < QR) sSum[tid] = 0u;
-  if (wave < nkc) load_k(wave, kn);
+  if (!HOLD && wave < nkc) load_k(wave, kn);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's part of the table
   __syncthreads();
   int32_t rowmax[QT];
@@ -190,15 +216,12 @@ void attn_prefill_split_kernel(AttnArgs a, int qtiles, int tiles, int per_xcd) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[u][t][r] = 0;
   }
-  for (int kc = wave; kc < nkc; kc += NW) {
-    v4i vf[KS];
-    load_v(kc, vf);
-    next_k(kc);
+  auto chunk_pv = [&](int kc, const v4i (&f)[KS], const v4i (&vf)[KS]) {
     auto chunk = [&](auto full_tag) {
       constexpr bool FULL = decltype(full_tag)::value;
 #pragma unroll
         for (int u = 0; u < QT; ++u) {
-          const v16i s = scores(kf, u);
+          const v16i s = scores(f, u);
           const ScoreIndex ix(a, rowmax[u]);
           uint32_t pb[16];
 #pragma unroll
@@ -240,6 +263,23 @@ void attn_prefill_split_kernel(AttnArgs a, int qtiles, int tiles, int per_xcd) {
       chunk(std::true_type{});
     else
       chunk(std::false_type{});
+  };
+  if constexpr (HOLD) {
+#pragma unroll
+    for (int i = 0; i < kHold; ++i) {
+      if (wave + NW * i < nkc) chunk_pv(wave + NW * i, kh[i], vh[i % kAhead]);
+      if (i + kAhead < kHold) {
+        load_v(min(wave + NW * (i + kAhead), nkc - 1), vh[i % kAhead]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  } else {
+    for (int kc = wave; kc < nkc; kc += NW) {
+      v4i vf[KS];
+      load_v(kc, vf);
+      next_k(kc);
+      chunk_pv(kc, kf, vf);
+    }
   }
 
   // ---- the waves' sums meet in LDS ----
@@ -271,11 +311,12 @@ void attn_prefill_split_kernel(AttnArgs a, int qtiles, int tiles, int per_xcd) {
   }
 }
 
-template <int KS, bool HAS_MASK, bool DF, int QT>
+template <int KS, bool HAS_MASK, bool DF, int QT, bool HOLD>
 int launch_split(const AttnArgs &a, hipStream_t s) {
+  constexpr int NW = HOLD ? 8 : 4;
   const int qtiles = (a.Tq + 32 * QT - 1) / (32 * QT);
   const int tiles = qtiles * a.H * a.B, per_xcd = (tiles + 7) / 8;
-  hipLaunchKernelGGL((attn_prefill_split_kernel<KS, HAS_MASK, DF, QT>), dim3((unsigned)(per_xcd * 8)), dim3(64 * NW),
+  hipLaunchKernelGGL((attn_prefill_split_kernel<KS, HAS_MASK, DF, QT, NW, HOLD>), dim3((unsigned)(per_xcd * 8)), dim3(64 * NW),
                      0, s, a, qtiles, tiles, per_xcd);
   return check_launch("attn_prefill_split_kernel");
 }
@@ -291,12 +332,19 @@ int launch_attn_prefill_split(const AttnArgs &a, hipStream_t s) {
   const int64_t per_head = (a.Tq + 31) / 32, tiles = per_head * a.H * a.B;
   if (tiles == 0) return 0;
   if (tiles > 0x3fffffffLL) return fail("attention grid too large");
-  const bool two = per_head > 2 && tiles > kSplitPairTiles;
-#define IW_PS(KS_, QT_)                                                        \
-  do {                                                                         \
-    if (a.mask) return launch_split<KS_, true, false, QT_>(a, s);              \
-    if (a.D == 32 * (KS_)) return launch_split<KS_, false, true, QT_>(a, s);   \
-    return launch_split<KS_, false, false, QT_>(a, s);                         \
+  const bool hold = a.Tk > 8 * KC && a.Tk <= 8 * kHold * KC && a.D <= 96 &&
+                    (a.D <= 64 ? per_head <= 2 || tiles <= 2 * kCus : tiles <= 4 * kCus);
+  const bool two = per_head > 2 && (tiles > kSplitPairTiles || (hold && tiles > kCus));
+#define IW_PN(KS_, QT_, HOLD_)                                                        \
+  do {                                                                                \
+    if (a.mask) return launch_split<KS_, true, false, QT_, HOLD_>(a, s);              \
+    if (a.D == 32 * (KS_)) return launch_split<KS_, false, true, QT_, HOLD_>(a, s);   \
+    return launch_split<KS_, false, false, QT_, HOLD_>(a, s);                         \
+  } while (0)
+#define IW_PS(KS_, QT_)             \
+  do {                              \
+    if (hold) IW_PN(KS_, QT_, true); \
+    IW_PN(KS_, QT_, false);         \
   } while (0)
   switch ((a.D + 31) / 32) {
     case 1:
@@ -310,6 +358,7 @@ int launch_attn_prefill_split(const AttnArgs &a, hipStream_t s) {
     default: return fail("fused attention supports head_dim <= 128");
   }
 #undef IW_PS
+#undef IW_PN
 }
 
 }  // namespace iw

@@ -498,6 +498,18 @@ def test_attention_prefill_tile_counts(iw, oracle, gpu, B, H, Tq, Tk, D, masked)
         assert np.array_equal(got, exp), shift
 
 
+# Eight waves that hold their K fragments: the first and last key counts of the
+# form, a last chunk of one key, one tile and pairs of tiles, with and without waves
+# that have no chunk left.
+@pytest.mark.parametrize("B,H,Tq,Tk,D", [(1, 3, 33, 256, 64), (1, 3, 33, 257, 64), (2, 3, 65, 1535, 64),
+                                         (1, 2, 96, 1536, 64), (1, 2, 40, 1537, 64), (4, 28, 70, 289, 64),
+                                         (30, 20, 5, 300, 64), (1, 4, 65, 1505, 96), (3, 20, 97, 520, 96),
+                                         (2, 3, 35, 700, 48), (1, 3, 65, 769, 32), (1, 2, 33, 600, 80)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_prefill_held_keys(iw, oracle, gpu, B, H, Tq, Tk, D, masked):
+    test_attention_prefill_tile_counts(iw, oracle, gpu, B, H, Tq, Tk, D, masked)
+
+
 def test_argmax_rows(iw, gpu):
     r = gen.rng(9)
     x = gen.i8(r, (7, 51865))
