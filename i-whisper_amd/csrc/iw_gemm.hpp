@@ -90,7 +90,7 @@ struct GemmArgs {
   void *out = nullptr;
   int64_t ldc = 0;
   int64_t out_T = 1;  // OUT_NCT: rows are (b, t) with t in [0, out_T)
-  LnRows ln;  // gemm_frag only: a is not used
+  LnRows ln;  // gemm_frag only; with ln.x set, a is not used
   // the next decode GEMM's weight, read into L2 (gemm_frag_kernel only)
   FragPrefetch pf;
   // per-tensor int8 epilogue (classifier) only, gemm_frag_kernel: the first

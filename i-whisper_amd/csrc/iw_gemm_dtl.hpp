@@ -5,7 +5,7 @@
 // channels-last input (+GeLU, + positional add_requant15).
 //
 // C[m][n] = sum_k A[m][k] * B[n][k], both operands K-contiguous int8.
-// Block tile 32 MI WM (M) x 32 NJ WN (N) x 64 (K); WM x WN waves, each an
+// Block tile 32 MI WM (M) x 32 NJ WN (N) x BK (K); WM x WN waves, each an
 // MI x NJ grid of v_mfma_i32_32x32x32_i8 blocks. The tile sizes in use and
 // the rule that picks one are in iw_gemm_dtl.hip.
 //
@@ -16,9 +16,10 @@
 // the release fence of __syncthreads() would drain every load and is not
 // used in the loop.
 //
-// LDS rows are 64 bytes (4 chunks of 16) with chunk c of row r stored at
-// position c ^ swz(r), swz(r) = 2*bit2(r) + (bit1(r) ^ bit3(r)), so that the
-// ds_read_b128 fragment reads of 8 or 16 consecutive rows hit distinct banks.
+// LDS rows are BK = 64 or 128 bytes (4 or 8 chunks of 16) with chunk c of row r
+// stored at position c ^ swz(r), swz(r) = 2*bit2(r) + (bit1(r) ^ bit3(r)) or
+// (r / 2) % 8, so that the ds_read_b128 fragment reads of 8 or 16 consecutive
+// rows hit distinct banks.
 //
 // The zero-point row sums sum_k A[m][k] are taken with v_dot4 from the A
 // fragments already in registers (the waves sharing rows split the
