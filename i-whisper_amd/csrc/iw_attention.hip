@@ -810,6 +810,13 @@ __global__ __launch_bounds__(64 * NWV) void attn_decode_cache_kernel(AttnArgs a,
 // tie (324 blocks: 17.1 and 17.8).
 constexpr int DM_NW = 16, DM_NR = 4, DM_CH = 256;
 constexpr int64_t kManyWavesMaxBlocks = 256;
+// The fused cross-attention from there to four blocks per CU: eight waves with the
+// same chunks and slots (two blocks per CU). us per token step with four and eight
+// waves: 264 / 324 / 504 blocks of 768 channels 725 -> 707, 737 -> 714, 753 -> 725; 500 / 800
+// of 1280 2160 -> 2081, 2547 -> 2491; 1024 of 1024 1957 -> 1912; 2560 4440 and 4439 (128-key chunks
+// or three slots are 0.2 to 6 % slower at all of them).
+constexpr int DH_NW = 8;
+constexpr int64_t kHalfWavesMaxBlocks = 1024;
 
 // the self-attention instance (at most 512 keys) has its own ring shape
 #ifndef IW_DSS_NR
@@ -1586,6 +1593,9 @@ int launch_attn_decode_cross_lnq(const AttnArgs &a, const LnQueryArgs &lq, hipSt
   const dim3 grid((unsigned)(a.B * a.H));
   if (grid.x <= kManyWavesMaxBlocks)
     hipLaunchKernelGGL((attn_decode_cross_lnq_kernel<DM_NR, DM_CH, DM_NW>), grid, dim3(64 * DM_NW), 0, s,
+                       a, lq);
+  else if (grid.x <= kHalfWavesMaxBlocks)
+    hipLaunchKernelGGL((attn_decode_cross_lnq_kernel<DM_NR, DM_CH, DH_NW>), grid, dim3(64 * DH_NW), 0, s,
                        a, lq);
   else
     hipLaunchKernelGGL((attn_decode_cross_lnq_kernel<IW_DS_NR, IW_DS_CH, 4>), grid, dim3(256), 0, s, a, lq);

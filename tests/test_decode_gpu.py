@@ -425,3 +425,11 @@ def test_attention_decode_cache_block_counts(iw, oracle, gpu, B, H, D, Tk):
 @pytest.mark.parametrize("B,H,Tk", [(1, 6, 1), (1, 8, 255), (20, 12, 257), (12, 20, 1500), (14, 20, 129)])
 def test_attention_decode_cross_lnq_block_counts(iw, oracle, gpu, B, H, Tk):
     test_attention_decode_cross_lnq(iw, oracle, gpu, B, H, Tk, True, True)
+
+
+# Two to four blocks per CU take eight waves per block: the edges of that range and of
+# the 256-key chunks.
+@pytest.mark.parametrize("B,H,Tk", [(33, 8, 1), (65, 16, 255), (86, 12, 257), (64, 16, 1500), (52, 20, 513),
+                                    (43, 6, 2048), (13, 20, 1500)])
+def test_attention_decode_cross_lnq_eight_waves(iw, oracle, gpu, B, H, Tk):
+    test_attention_decode_cross_lnq(iw, oracle, gpu, B, H, Tk, True, True)
