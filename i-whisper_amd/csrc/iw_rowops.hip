@@ -691,9 +691,11 @@ __global__ __launch_bounds__(GF_NT) void greedy_filtered_kernel(const int8_t *__
   const bool lps = f.sum_logprobs != nullptr;
   float st_sum = 0.f, sx = 0.f;
   if (lps || (rules && ks != 0)) {
+    // rounded once: every logit of a value takes the same entry, so an error of it
+    // would not average out over the row
     if (tid < 256) {
-      s_et[tid] = expf((float)(tid - 128 - mt) * f.scale);
-      s_ex[tid] = expf((float)(tid - 128 - mxt) * f.scale);
+      s_et[tid] = (float)exp((double)(tid - 128 - mt) * (double)f.scale);
+      s_ex[tid] = (float)exp((double)(tid - 128 - mxt) * (double)f.scale);
     }
     __syncthreads();
     visit([&](int, const uint32_t (&ws)[4], uint32_t tb, uint32_t sb) {
