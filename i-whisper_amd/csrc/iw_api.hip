@@ -596,13 +596,14 @@ int iw_shift_exp_table(uint8_t *table, int32_t frac_bits, iw_stream_t stream) {
   return launch_shift_exp_lut(table, frac_bits, as_stream(stream));
 }
 
-int iw_attention(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, int64_t k_sb,
-                 int64_t k_sh, int64_t k_st, const int8_t *vt, int64_t v_sb, int64_t v_sh,
-                 int64_t v_sd, int8_t *out, int64_t o_sb, int64_t o_st, const bool *mask,
-                 int64_t batch, int64_t heads, int64_t q_length, int64_t k_length,
-                 int64_t head_dim, uint8_t qk_multiplier, int8_t qk_shift, int32_t frac_bits,
-                 uint8_t av_multiplier, int8_t av_shift, uint32_t rsqrt_offset,
-                 const uint8_t *table, bool decode, iw_stream_t stream) {
+int iw_attention_strided_mask(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, int64_t k_sb,
+                              int64_t k_sh, int64_t k_st, const int8_t *vt, int64_t v_sb, int64_t v_sh,
+                              int64_t v_sd, int8_t *out, int64_t o_sb, int64_t o_st, const bool *mask,
+                              int64_t mask_ld, int64_t batch, int64_t heads, int64_t q_length,
+                              int64_t k_length, int64_t head_dim, uint8_t qk_multiplier, int8_t qk_shift,
+                              int32_t frac_bits, uint8_t av_multiplier, int8_t av_shift,
+                              uint32_t rsqrt_offset, const uint8_t *table, bool decode,
+                              iw_stream_t stream) {
   IW_REQUIRE(frac_bits > 0 && frac_bits < 14, "frac_bits must be in [1, 14)");
   IW_REQUIRE(rsqrt_offset <= 29, "rsqrt_offset must be in [0,29]");
   IW_REQUIRE(head_dim > 0 && head_dim <= 128 && head_dim % 16 == 0,
@@ -610,6 +611,7 @@ int iw_attention(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, i
   IW_REQUIRE(batch >= 0 && heads > 0 && q_length >= 0 && k_length >= 0, "invalid attention shape");
   IW_REQUIRE(batch <= 0x7fffffff && q_length <= 0x7fffffff && k_length <= 0x7fffffff,
              "attention shape too large");
+  IW_REQUIRE(!mask || mask_ld >= k_length, "mask rows must hold k_length keys");
   if (batch * q_length == 0) return IW_OK;
   IW_REQUIRE(q && k && vt && out, "null tensor pointer");
   IW_REQUIRE(v_sd % 16 == 0 && v_sd >= ((k_length + 15) / 16) * 16,
@@ -636,6 +638,7 @@ int iw_attention(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, i
   a.o_sb = o_sb;
   a.o_st = o_st;
   a.mask = reinterpret_cast<const uint8_t *>(mask);
+  a.mask_ld = mask_ld;
   a.B = (int32_t)batch;
   a.H = (int32_t)heads;
   a.Tq = (int32_t)q_length;
@@ -663,6 +666,18 @@ int iw_attention(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, i
       cus = v;
   }
   return launch_attn_prefill(a, cus * 4, as_stream(stream));
+}
+
+int iw_attention(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, int64_t k_sb,
+                 int64_t k_sh, int64_t k_st, const int8_t *vt, int64_t v_sb, int64_t v_sh,
+                 int64_t v_sd, int8_t *out, int64_t o_sb, int64_t o_st, const bool *mask,
+                 int64_t batch, int64_t heads, int64_t q_length, int64_t k_length,
+                 int64_t head_dim, uint8_t qk_multiplier, int8_t qk_shift, int32_t frac_bits,
+                 uint8_t av_multiplier, int8_t av_shift, uint32_t rsqrt_offset,
+                 const uint8_t *table, bool decode, iw_stream_t stream) {
+  return iw_attention_strided_mask(q, q_sb, q_st, k, k_sb, k_sh, k_st, vt, v_sb, v_sh, v_sd, out, o_sb, o_st, mask,
+                                   k_length, batch, heads, q_length, k_length, head_dim, qk_multiplier, qk_shift,
+                                   frac_bits, av_multiplier, av_shift, rsqrt_offset, table, decode, stream);
 }
 
 int iw_transpose_heads(const int8_t *src, int64_t src_sb, int64_t src_st, int8_t *dst,

@@ -321,7 +321,7 @@ void attn_prefill_kernel(AttnArgs a) {
           for (int r = 0; r < 16; ++r) {
             const int key = kbase0 + r;
             bool ok = key < a.Tk;
-            if (HAS_MASK) ok = ok && q < a.Tq && !a.mask[(int64_t)q * a.Tk + key];
+            if (HAS_MASK) ok = ok && q < a.Tq && !a.mask[q * a.mask_ld + key];
             if (ok) mx = max(mx, s[r]);
           }
         }
@@ -380,7 +380,7 @@ void attn_prefill_kernel(AttnArgs a) {
           if constexpr (!FULL) {
             const int key = kbase0 + r;
             bool ok = key < a.Tk;
-            if (HAS_MASK) ok = ok && q < a.Tq && !a.mask[(int64_t)q * a.Tk + key];
+            if (HAS_MASK) ok = ok && q < a.Tq && !a.mask[q * a.mask_ld + key];
             pb[r] &= ok ? 0xffu : 0u;
           }
         }
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
       }
     }
     sS[j] = acc;
-    const bool ok = !(a.mask && a.mask[(int64_t)qi * a.Tk + j]);
+    const bool ok = !(a.mask && a.mask[qi * a.mask_ld + j]);
     if (ok) mx = max(mx, acc);
   }
 #pragma unroll
@@ -516,7 +516,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
   uint32_t psum = 0, hi = 0;
   for (int j = tid; j < a.Tk; j += 256) {
     uint32_t p = 0;
-    if (!(a.mask && a.mask[(int64_t)qi * a.Tk + j])) {
+    if (!(a.mask && a.mask[qi * a.mask_ld + j])) {
       const int32_t h16 = qk_requant16(sS[j], a.qk_m, a.qk_s);
       // x_sub = qk - rmp1 modulo 2^16
       p = shift_exp_one((int32_t)(int16_t)(uint16_t)((uint32_t)h16 - rmp1), a.frac_bits);

@@ -136,7 +136,7 @@ void attn_prefill_split_kernel(AttnArgs a, int qtiles, int tiles, int per_xcd) {
   auto counts = [&](int u, int key) {
     const int q = q0 + 32 * u;
     bool ok = key < Tk;
-    if (HAS_MASK) ok = ok && q < a.Tq && !a.mask[(int64_t)q * Tk + key];
+    if (HAS_MASK) ok = ok && q < a.Tq && !a.mask[q * a.mask_ld + key];
     return ok;
   };
 

@@ -27,7 +27,8 @@ struct AttnArgs {
   int64_t v_sq = 4;  // key-quad stride; 4 = transposed rows
   int8_t *out = nullptr;
   int64_t o_sb = 0, o_st = 0;
-  const uint8_t *mask = nullptr;  // [Tq][Tk] bool bytes, or null
+  const uint8_t *mask = nullptr;  // [Tq][Tk] bool bytes with mask_ld between rows, or null
+  int64_t mask_ld = 0;
   int32_t B = 0, H = 0, Tq = 0, Tk = 0, D = 0;
   uint32_t qk_m = 0;   // uint8 multiplier
   uint32_t qk_s = 0;   // shift clamped at 0

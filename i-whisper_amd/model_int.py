@@ -336,12 +336,7 @@ class MultiHeadAttention_int(_ScalarCache, nn.Module):
         if mask is not None:  # model_int.py:786-799
             q_offset = Tk - Tq
             assert q_offset >= 0
-            slices = getattr(mask, "attn_slices", None)  # one copy per decoder call, not one per layer
-            attn_mask = None if slices is None else slices.get((Tq, Tk))
-            if attn_mask is None:
-                attn_mask = mask[q_offset:q_offset + Tq, :Tk].contiguous()
-                if slices is not None:
-                    slices[Tq, Tk] = attn_mask
+            attn_mask = mask[q_offset:q_offset + Tq, :Tk]
         s = self._scalars()
         out = torch.empty((B, Tq, C), dtype=torch.int8, device=q.device)
         if D % 16 == 0 and D <= 128 and Tk <= 4096:
@@ -355,9 +350,15 @@ class MultiHeadAttention_int(_ScalarCache, nn.Module):
             tp = vt.shape[-1]
             decode = Tq <= 8
             table = None if decode else self.shift_exp_table()
-            _lib.call("iw_attention", q.data_ptr(), Tq * C, C, k.data_ptr(), Tk * C, D, C,
+            ld = Tk
+            if attn_mask is not None:  # read in place where its rows are whole bytes side by side
+                if attn_mask.element_size() != 1 or attn_mask.stride(1) != 1 or attn_mask.stride(0) < Tk:
+                    attn_mask = attn_mask.contiguous()
+                else:
+                    ld = attn_mask.stride(0)
+            _lib.call("iw_attention_strided_mask", q.data_ptr(), Tq * C, C, k.data_ptr(), Tk * C, D, C,
                       vt.data_ptr(), H * D * tp, D * tp, tp, out.data_ptr(), Tq * C, C,
-                      _ptr(attn_mask), B, H, Tq, Tk, D, s["qm"], s["qs"], s["f"], s["am"],
+                      _ptr(attn_mask), ld, B, H, Tq, Tk, D, s["qm"], s["qs"], s["f"], s["am"],
                       s["as_"], self.rsqrt_offset, _ptr(table), decode, _stream())
             return out
         # Other head sizes: the three reference ops, each on the GPU.
@@ -368,6 +369,7 @@ class MultiHeadAttention_int(_ScalarCache, nn.Module):
         rm = torch.empty((B, H, Tq, 1), dtype=torch.int16, device=q.device)
         p = torch.empty((B, H, Tq, Tk), dtype=torch.uint8, device=q.device)
         rs = torch.empty((B, H, Tq, 1), dtype=torch.int32, device=q.device)
+        attn_mask = None if attn_mask is None else attn_mask.contiguous()
         mp = _ptr(attn_mask)
         _lib.call("iw_qk_requant_rowmax", qh.data_ptr(), kh.data_ptr(), mp, qk.data_ptr(),
                   rm.data_ptr(), B, H, Tq, Tk, D, s["qm"], s["qs"], mp is not None, _stream())
@@ -631,11 +633,8 @@ class TextDecoder_int(nn.Module):
             if lo < 0 or hi >= self.n_vocab:
                 raise RuntimeError("token id out of range")
         x = self.embed(x, offset)
-        # a view of its own, which carries the slice that the layers of this call share
-        mask = self.mask.view(self.mask.shape)
-        mask.attn_slices = {}
         for block in self.blocks:
-            x = block(x, xa, mask=mask, kv_cache=kv_cache)
+            x = block(x, xa, mask=self.mask, kv_cache=kv_cache)
         h = self.ln.normalize(x)
         alpha = self.act_logits_alpha.detach()
         if not self.dequant_need:

@@ -230,6 +230,17 @@ int iw_attention(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, i
                  uint8_t av_multiplier, int8_t av_shift, uint32_t rsqrt_offset,
                  const uint8_t *table, bool decode, iw_stream_t stream);
 
+/* iw_attention over a mask whose rows lie mask_ld >= k_length bytes apart, so that a slice of
+ * a larger mask (the decoder's [n_ctx, n_ctx] one, model_int.py:786-799) is read where it is. */
+int iw_attention_strided_mask(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, int64_t k_sb,
+                              int64_t k_sh, int64_t k_st, const int8_t *vt, int64_t v_sb, int64_t v_sh,
+                              int64_t v_sd, int8_t *out, int64_t o_sb, int64_t o_st, const bool *mask,
+                              int64_t mask_ld, int64_t batch, int64_t heads, int64_t q_length,
+                              int64_t k_length, int64_t head_dim, uint8_t qk_multiplier, int8_t qk_shift,
+                              int32_t frac_bits, uint8_t av_multiplier, int8_t av_shift,
+                              uint32_t rsqrt_offset, const uint8_t *table, bool decode,
+                              iw_stream_t stream);
+
 /* Layout helpers for the KV caches (the reference's view/permute/.contiguous()
  * copies and hook-side torch.cat, model_int.py:842-949 and 1604-1610):
  * transpose_heads writes, with p = t_offset + t,

@@ -422,6 +422,31 @@ def test_attention_decode_block_counts(iw, oracle, gpu, B, H, Tq, Tk):
     test_attention_decode_fused(iw, oracle, gpu, B, H, Tq, Tk, 64, False)
 
 
+# A slice of a larger mask, read where it is, in each kernel that takes one: one query row per
+# block, 32-query tiles (with and without the chunks held) and 128-query tiles.
+@pytest.mark.parametrize("B,H,Tq,Tk,D", [(2, 3, 3, 17, 64), (1, 2, 8, 2100, 96), (1, 3, 70, 150, 64),
+                                         (2, 3, 33, 300, 96), (20, 28, 65, 70, 64)])
+def test_attention_strided_mask(iw, oracle, gpu, B, H, Tq, Tk, D):
+    _print_case("attention strided mask", B, H, Tq, Tk, D)
+    q, k, v, qm, qs, f, am, as_ = gen.attn_case(B + Tq + Tk, B, H, Tq, Tk, D)
+    full = gen.rng(Tk).random((Tq + 3, Tk + 21)) < 0.4
+    part = T(full)[2:2 + Tq, 5:5 + Tk]
+    exp = oracle.attention(q, k, v, np.ascontiguousarray(full[2:2 + Tq, 5:5 + Tk]), qm, qs, f, am, as_)
+    C, pad, decode = H * D, (Tk + 15) // 16 * 16, Tq <= 8
+    qt, kt = (T(a.transpose(0, 2, 1, 3).reshape(B, -1, C)) for a in (q, k))
+    vt = T(np.pad(v, ((0, 0), (0, 0), (0, 0), (0, pad - Tk))))
+    out = torch.empty((B, Tq, C), dtype=torch.int8, device="cuda")
+    args = [qt.data_ptr(), Tq * C, C, kt.data_ptr(), Tk * C, D, C, vt.data_ptr(), C * pad, D * pad, pad,
+            out.data_ptr(), Tq * C, C, part.data_ptr()]
+    table = None if decode else iw.kernels.shift_exp_table_hip(f)
+    tail = [B, H, Tq, Tk, D, qm, qs, f, am, as_, 16, None if decode else table.data_ptr(), decode,
+            torch.cuda.current_stream().cuda_stream]
+    iw._lib.call("iw_attention_strided_mask", *args, part.stride(0), *tail)
+    assert np.array_equal(host(out), exp)
+    with pytest.raises(RuntimeError, match="mask rows"):
+        iw._lib.call("iw_attention_strided_mask", *args, Tk - 1, *tail)
+
+
 @pytest.mark.parametrize("decode", [False, True])
 def test_attention_fused_wrap_corner(iw, oracle, gpu, decode):
     """Scores saturating at +32767 wrap rmp1 and give P = 128 at x_sub = 0."""

@@ -110,6 +110,42 @@ def test_decoder_reference_style_cache(iw, small):
     assert np.array_equal(host(got), exp)
 
 
+@pytest.mark.parametrize("n_tok", [4, 12])
+def test_decoder_layers_read_the_mask_themselves(iw, small, n_tok):
+    """Every layer is handed the decoder's own mask and reads it as it is when the layer runs: a
+    forward hook of the first layer that edits it is seen by the second."""
+    dims, P, model, ref = small
+    dec = model.decoder
+    xa = T(ref.encoder(iw.synth.synthetic_mel(2, dims.n_mels, 2 * dims.n_audio_ctx, seed=33)))
+    toks = T(gen.rng(n_tok).integers(0, dims.n_vocab, size=(2, n_tok)).astype(np.int64))
+    before = dec.mask.clone()
+    after = before.clone()
+    after[n_tok // 2:, : n_tok // 2] = True
+    handed = []
+    hooks = [b.register_forward_pre_hook(lambda mod, args, kw: handed.append(kw["mask"]), with_kwargs=True)
+             for b in dec.blocks]
+
+    def edit(mod, args, out):
+        dec.mask.copy_(after)
+
+    hooks.append(dec.blocks[0].register_forward_hook(edit))
+    try:
+        with torch.no_grad():
+            plain = dec.blocks[1](dec.blocks[0](dec.embed(toks, 0), xa, mask=before), xa, mask=before)
+            dec.mask.copy_(before)
+            del handed[:]
+            got = dec(toks, xa)
+            assert all(m is dec.mask for m in handed) and len(handed) == 2
+            x = dec.blocks[1](dec.blocks[0](dec.embed(toks, 0), xa, mask=before), xa, mask=after)
+            exp = dec.classify(dec.ln.normalize(x)).float().div(dec.act_logits_alpha)
+    finally:
+        for h in hooks:
+            h.remove()
+        dec.mask.copy_(before)
+    assert not torch.equal(plain, x)  # the edit matters
+    assert torch.equal(got, exp)
+
+
 @pytest.mark.parametrize("batch,steps", [(1, 6), (3, 10)])
 def test_greedy_decode_runner(iw, small, batch, steps):
     dims, P, model, ref = small
