@@ -629,7 +629,8 @@ class TextDecoder_int(nn.Module):
         check_backend(self.backend)
         offset = next(iter(kv_cache.values())).shape[1] if kv_cache else 0
         if x.numel():
-            lo, hi = torch.stack(torch.aminmax(x)).tolist()  # one read of the device
+            # one read of the device; int() as for each value on its own (NaN is refused)
+            lo, hi = map(int, torch.stack(torch.aminmax(x)).tolist())
             if lo < 0 or hi >= self.n_vocab:
                 raise RuntimeError("token id out of range")
         x = self.embed(x, offset)

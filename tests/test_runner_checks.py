@@ -50,3 +50,21 @@ def test_greedy_decode_rejects_runner_with_other_filters(iw):
     prompt = torch.zeros((4, 3), dtype=torch.int64)
     with pytest.raises(ValueError, match="filters"):
         iw.greedy_decode(model, torch.zeros((4, 1500, 384), dtype=torch.int8), prompt, 5, runner=runner)
+
+
+@pytest.mark.parametrize("tokens,error", [([1.0, float("nan")], ValueError), ([float("inf"), 1.0], OverflowError),
+                                          ([float("-inf"), 1.0], OverflowError), ([1, 100], RuntimeError),
+                                          ([-1, 5], RuntimeError), ([0.5, -1.0], RuntimeError),
+                                          ([0, 99], None), ([True, False], None), ([-0.5, 99.5], None)])
+def test_decoder_forward_checks_tokens(iw, tokens, error):
+    """Values that are no token of the vocabulary are refused before the embedding gather reads a
+    row of the table for them; those that convert to one are passed on."""
+    class Reached(Exception):
+        pass
+
+    def embed(*args):
+        raise Reached
+
+    dec = SimpleNamespace(backend="hip", n_vocab=100, embed=embed)
+    with pytest.raises(error or Reached):
+        iw.TextDecoder_int.forward(dec, torch.tensor([tokens]), None)
