@@ -640,7 +640,9 @@ class TextDecoder_int(nn.Module):
         alpha = self.act_logits_alpha.detach()
         if not self.dequant_need:
             return self.classify(h)
-        if alpha.numel() == 1 and alpha.dim() <= 3 and alpha.dtype == torch.float32 and alpha.device == h.device:
+        # with this class's own classify, which the one call restates
+        if (getattr(self.classify, "__func__", None) is _OWN_CLASSIFY and alpha.numel() == 1 and alpha.dim() <= 3
+                and alpha.dtype == torch.float32 and alpha.device == h.device):
             return self._classify_dequant(h, alpha)
         return self.classify(h).float().div(alpha)
 
@@ -651,6 +653,8 @@ class TextDecoder_int(nn.Module):
         new.load_state_dict(quant_layer.state_dict())
         return new
 
+
+_OWN_CLASSIFY = TextDecoder_int.classify
 
 QUANT_MODULES = [Conv1d_int, GELU_int, LayerNorm_int, AudioEncoder_int, TextDecoder_int,
                  ResidualAttentionBlock_int, MultiHeadAttention_int]

@@ -68,3 +68,23 @@ def test_decoder_forward_checks_tokens(iw, tokens, error):
     dec = SimpleNamespace(backend="hip", n_vocab=100, embed=embed)
     with pytest.raises(error or Reached):
         iw.TextDecoder_int.forward(dec, torch.tensor([tokens]), None)
+
+
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+def test_decoder_forward_calls_an_overridden_classify(iw, monkeypatch, how):
+    """forward divides what classify returns, also where a program has put its own in its place."""
+    def classify(self, h):
+        return torch.full((*h.shape[:2], self.n_vocab), 7, dtype=torch.int8)
+
+    cls = iw.TextDecoder_int
+    if how == "subclass":
+        cls = type("Decoder", (cls,), {"classify": classify})
+    elif how == "class":
+        monkeypatch.setattr(cls, "classify", classify)
+    dec = cls(n_vocab=20, n_ctx=8, n_state=384, n_head=6, n_layer=0)
+    if how == "instance":
+        dec.classify = lambda h: classify(dec, h)
+    dec.embed = lambda x, offset: torch.zeros((*x.shape, 384), dtype=torch.int16)
+    dec.ln.normalize = lambda x: x.to(torch.int8)
+    dec.act_logits_alpha.data.fill_(2.0)
+    assert torch.equal(dec(torch.tensor([[1, 2, 3]]), None), torch.full((1, 3, 20), 3.5))
