@@ -160,9 +160,10 @@ __device__ __forceinline__ int32_t wave_max_dpp(int32_t v) {
 // global_load_lds_dwordx4: lane l copies 16 bytes from src to LDS byte
 // address lds + 16 l (lds wave-uniform). Inline assembly, so that the
 // compiler adds no waits for it: its users wait on vmcnt themselves. No
-// kernel using it keeps a value in M0.
+// kernel using it keeps a value in M0. The load needs a wait state after M0 is
+// written, which the compiler does not insert within inline assembly.
 __device__ __forceinline__ void dma16_lds(const int8_t *src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds)
                : "memory", "m0");
 }
 #pragma clang diagnostic pop

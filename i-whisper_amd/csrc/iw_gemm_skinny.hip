@@ -38,11 +38,12 @@ constexpr int SK = 128;    // K bytes per stage (one LDS row)
 // One 16-byte global -> LDS copy per lane (global_load_lds_dwordx4): the wave
 // writes 1 KB at LDS byte address `lds` (lane l at lds + 16 l). Issued as
 // inline assembly so that the compiler adds no waits for it; the loop waits
-// on vmcnt itself. No kernel using it keeps a value in M0.
+// on vmcnt itself. No kernel using it keeps a value in M0. (s_nop: see
+// dma16_lds of iw_common.hpp.)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(const int8_t *src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds)
                : "memory", "m0");
 }
 #pragma clang diagnostic pop

@@ -4,6 +4,8 @@ header's argument counts, and argument validation reports errors through
 iw_last_error() before any device work."""
 import ctypes
 import re
+import shutil
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -76,3 +78,25 @@ def test_frag_bytes(iw):
     assert v("iw_frag_bytes", 33, 5120) == 64 * 5120
     assert v("iw_frag_bytes", 51865, 1280) == 51872 * 1280
     assert v("iw_frag_bytes", 1, 5121) == 0 and v("iw_frag_bytes", -1, 4) == 0
+
+
+def test_lds_loads_keep_their_wait_state(lib, tmp_path):
+    """A load into LDS takes its address from M0 and needs one wait state after a write of it. The
+    compiler inserts none within inline assembly, so the built kernels are looked through."""
+    objdump = Path("/opt/rocm/llvm/bin/llvm-objdump")
+    if not objdump.exists():
+        pytest.skip("no llvm-objdump")
+    shutil.copy(lib._name, tmp_path / "lib.so")
+    subprocess.run([objdump, "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
+    loads, bad = 0, []
+    for code in tmp_path.glob("*gfx950*"):
+        out = subprocess.run([objdump, "-d", "--no-show-raw-insn", code], check=True, capture_output=True, text=True)
+        before = ""
+        for line in out.stdout.splitlines():
+            op = line.split("//")[0].strip()
+            if re.match(r"(global|buffer|scratch)_load_lds", op):
+                loads += 1
+                if re.match(r"s_\w+ m0\b", before):
+                    bad.append(op)
+            before = op
+    assert loads > 0 and not bad
