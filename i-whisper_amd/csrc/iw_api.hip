@@ -665,7 +665,7 @@ int iw_attention_strided_mask(const int8_t *q, int64_t q_sb, int64_t q_st, const
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
       cus = v;
   }
-  return launch_attn_prefill(a, cus * 4, as_stream(stream));
+  return launch_attn_prefill(a, cus * (head_dim <= 64 ? 4 : 3), as_stream(stream));
 }
 
 int iw_attention(const int8_t *q, int64_t q_sb, int64_t q_st, const int8_t *k, int64_t k_sb,

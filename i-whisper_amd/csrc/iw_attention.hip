@@ -152,7 +152,7 @@ __device__ __forceinline__ int key_row(int kk) {
 // DF: the head dim is exactly 32 KS, so whole-chunk K / V^T copies need no
 // bounds tests.
 template <int KS, bool HAS_MASK, bool DF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KS <= 2 ? 4 : 1)))
 void attn_prefill_kernel(AttnArgs a) {
   constexpr int DP = KS * 32;           // padded head dim
   // K and V^T rows of 4 chunks of 16 bytes (head_dim 64) are unpadded, with
@@ -1569,7 +1569,9 @@ int launch_attn_prefill(const AttnArgs &a, int max_blocks, hipStream_t s) {
   switch (ks) {
     case 1: IW_PF(1) break;
     case 2: IW_PF(2) break;
-    default: return fail("this prefill kernel takes head_dim <= 64");
+    case 3: IW_PF(3) break;
+    case 4: IW_PF(4) break;
+    default: return fail("fused attention supports head_dim <= 128");
   }
 #undef IW_PF
   return check_launch("attn_prefill_kernel");

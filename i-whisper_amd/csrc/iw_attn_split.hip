@@ -11,6 +11,7 @@
 // before the shift-exponential, and at the end the integer sums of P and P.V,
 // which are exact modulo 2^32 in any order. The arithmetic per score is
 // that of attn_prefill_kernel.
+#include <algorithm>
 #include <type_traits>
 
 #include "iw_attn_dev.hpp"
@@ -24,27 +25,38 @@ namespace {
 constexpr int KC = 32;  // keys per chunk
 constexpr int kHold = 6, kAhead = 3;  // chunks of a wave whose K it holds, V^T chunks ahead
 
-// Where this kernel runs (tiles of 32 queries; measured against 128 queries
-// per block, us):
-// * head_dim above 64 always: 4 heads of 96 over 1500 positions 98 -> 18.7 at
-//   batch 1, 230 -> 144 at batch 16 (the other kernel's registers leave it
-//   two blocks per CU).
-// * up to two tiles per head always, where 128 rows are mostly padding: 3
-//   masked queries of 2560 heads 30 -> 18.7, 12 queries of 2560 heads over
-//   1500 keys 194 -> 165.
-// * else up to kSplitMaxTiles tiles: 8 heads over 1500 positions 38 -> 22.7
-//   (376 tiles) and 39 -> 31.9 (752), 117 queries of 48 heads over 1500 keys
-//   38.6 -> 16.9; at 1880 tiles both take 57. Above that every SIMD has its
-//   waves either way, and four times the K / V^T reads per query cost more
-//   (376 -> 22.7, 7520 -> 226 against 164).
+// Where this kernel runs: attn_prefill_split_eligible, over tiles of 32 queries and the 128-query
+// blocks that the other kernel would have. Timed against each other at 12 .. 5120 heads,
+// 3 .. 1500 queries and 32 .. 2000 keys; us of the 128-query kernel and of this one:
+// * one tile per head always: 3 masked queries of 2560 heads 30 / 18.7, 12 queries of 2560 heads
+//   over 300 keys 53 / 34, over 1500 keys 194 / 140.
+// * two tiles per head: 64 queries of 400 heads over 300 keys 19.9 / 17.1, of 1600 heads 46.9 / 43.4.
+//   Not above 1024 tiles where the other kernel's 64-key chunks have no padding (2560 heads over
+//   448 keys 68 / 77, 1024 heads over 64 keys 16.1 / 18.1), nor above kSplitMaxTiles with more than
+//   768 keys (2560 heads over 1500 keys 207 / 259): there its one copy of K, V^T and the table serves
+//   64 queries instead of 32.
+// * more tiles per head: up to kSplitPairTiles (8 heads over 1500 positions 38 / 22.7, 376 tiles),
+//   above that, where a wave takes two tiles, up to two blocks per CU (20 heads over 1500 positions
+//   42.1 / 35.6), and up to three from 1000 keys on (324 heads of 128 queries over 1000 keys
+//   41.5 / 37.5, over 300 keys 20.3 / 22.9; 192 heads of 200 queries over 200 keys 19.0 / 20.4). The
+//   third block waits for the registers of the first two, and the chip is full either way.
+//   Masked rows cost the other kernel its short loops (192 heads of 256: 69.6 / 56.6), except where
+//   two chunks hold all keys (400 heads of 96: 31 / 40).
+// * head_dim up to 32: the other kernel's chunks are half as long, so its padded rows weigh more
+//   (64 heads of 32 over 750 positions 27.7 / 23.0, 1024 heads of 60 queries over 1500 keys 71 / 46).
+// * head_dim above 64, whose registers leave the other kernel two blocks per CU: always (4 heads
+//   of 96 over 1500 positions 98 / 18.7), except many full 128-query blocks that come out even on
+//   the CUs over few keys (1024 heads, 128 queries and keys: 46.7 / 61.0 at 96, 52.3 / 72.7 at 128;
+//   512 heads of 128, 256 of each: 69.6 / 91.0).
 // Above kSplitPairTiles (three blocks per CU) a wave takes two tiles over one
 // set of K / V^T fragments: 940 tiles 42.1 -> 35.6, 1504 tiles 55.2 -> 46.9.
-// Eight waves that hold their K fragments (HOLD) for 9 .. 48 chunks of keys, us with
-// four waves and with eight: 117 queries of 48 heads over 1500 keys (192 tiles)
-// 15.7 -> 11.7, 8 heads over 1500 positions (376; pairs, one block per CU) 22.5 -> 18.1, 12
-// queries of 320 / 2560 heads 24.5 -> 23.2 / 166 -> 146, 4 heads of 96 (188) 18.9 -> 15.8 and 16
-// (752) 53 -> 43; not at 564 tiles of 64 (30.5 / 31.7), 64 heads of 96 (144 / 161), 117 keys
-// (9.6 / 12.2: the chunks past the last are read for nothing) or head_dim 128 (spills).
+// Eight waves that hold their K fragments (HOLD) for 9 .. 48 chunks of keys: a wave loads six
+// chunks whether it has them or not, so this pays while a block has a CU to itself (117
+// queries of 48 heads over 1500 keys, us with four waves and with eight: 15.7 / 11.7; 8 heads over
+// 1500 positions 22.5 / 18.1; 4 heads of 96 18.9 / 15.8), and beyond only with most of the six
+// real: 12 queries of 2560 heads over 300 / 600 / 1500 keys 34 / 58, 55 / 75 and 166 / 140, 16 heads
+// of 96 over 1500 positions 53 / 43, 512 heads of 96 with 64 queries over 500 keys 31.7 / 46.5. Not at
+// head_dim 128, where it would spill.
 constexpr int64_t kSplitMaxTiles = 1600, kSplitPairTiles = 768, kCus = 256;
 
 // QT: 32-query subtiles per wave, all over the same K and V^T fragments.
@@ -324,16 +336,37 @@ int launch_split(const AttnArgs &a, hipStream_t s) {
 }  // namespace
 
 bool attn_prefill_split_eligible(const AttnArgs &a) {
-  const int64_t per_head = (a.Tq + 31) / 32;
-  return a.D > 64 || per_head <= 2 || per_head * a.H * a.B <= kSplitMaxTiles;
+  const int64_t heads = (int64_t)a.H * a.B, per_head = (a.Tq + 31) / 32, tiles = per_head * heads;
+  if (per_head == 1) return true;
+  // the other kernel's 64-key chunks hold next to no padding
+  const bool whole = (64 - a.Tk % 64) % 64 * 24 < a.Tk;
+  if (a.D > 64) {
+    const int64_t blocks = (a.Tq + 127) / 128 * heads, over = blocks % kCus;
+    const bool filled = (per_head % 4 == 0 || per_head % 4 == 3 || per_head > 8) && per_head > 3;
+    const bool even = blocks > kCus + kCus / 2 && (over == 0 || over > kCus / 2);
+    return !(filled && even && (a.D <= 96 ? a.Tk <= 128 : !a.mask && (a.Tk <= 128 || (whole && a.Tk <= 256))));
+  }
+  if (a.D <= 32) return per_head == 2 ? tiles <= 4 * kCus || a.Tk > 64 : tiles <= kSplitMaxTiles;
+  if (per_head == 2)
+    return tiles <= 4 * kCus || a.mask || (a.Tk <= 768 ? !whole : tiles <= kSplitMaxTiles);
+  if (tiles <= kSplitPairTiles) return true;
+  if (tiles > kSplitMaxTiles) return false;
+  const int64_t pairs = (per_head + 1) / 2 * heads;
+  return pairs <= 2 * kCus || (a.mask ? pairs <= 3 * kCus || a.Tk > 128 : pairs <= 3 * kCus && a.Tk >= 1000);
 }
 
 int launch_attn_prefill_split(const AttnArgs &a, hipStream_t s) {
   const int64_t per_head = (a.Tq + 31) / 32, tiles = per_head * a.H * a.B;
   if (tiles == 0) return 0;
   if (tiles > 0x3fffffffLL) return fail("attention grid too large");
-  const bool hold = a.Tk > 8 * KC && a.Tk <= 8 * kHold * KC && a.D <= 96 &&
-                    (a.D <= 64 ? per_head <= 2 || tiles <= 2 * kCus : tiles <= 4 * kCus);
+  const bool wide = a.D > 64;
+  const int64_t pairs = (per_head + 1) / 2 * (int64_t)a.H * a.B;
+  const bool hold =
+      a.Tk > 8 * KC && a.Tk <= 8 * kHold * KC && a.D <= 96 &&
+      (tiles <= kCus || (!wide && per_head > 2 && pairs <= kCus) ||
+       (a.Tk > 960 && (wide ? tiles <= 3 * kCus : per_head > 2 && tiles <= 2 * kCus)) ||
+       (a.Tk > 1200 && (wide ? tiles <= 4 * kCus
+                             : per_head == 1 || (per_head == 2 && (a.D <= 32 || tiles <= 5 * kCus)))));
   const bool two = per_head > 2 && (tiles > kSplitPairTiles || (hold && tiles > kCus));
 #define IW_PN(KS_, QT_, HOLD_)                                                        \
   do {                                                                                \
@@ -354,7 +387,7 @@ int launch_attn_prefill_split(const AttnArgs &a, hipStream_t s) {
       if (two) IW_PS(2, 2);
       IW_PS(2, 1);
     case 3: IW_PS(3, 1);
-    case 4: IW_PS(4, 1);
+    case 4: IW_PN(4, 1, false);
     default: return fail("fused attention supports head_dim <= 128");
   }
 #undef IW_PS

@@ -535,6 +535,58 @@ def test_attention_prefill_held_keys(iw, oracle, gpu, B, H, Tq, Tk, D, masked):
     test_attention_prefill_tile_counts(iw, oracle, gpu, B, H, Tq, Tk, D, masked)
 
 
+def _copies(n, *arrays):
+    """Batch rows repeated n times: as many heads as a large batch has, at a few heads' cost in the oracle."""
+    return [np.tile(x, (n, 1, 1, 1)) for x in arrays]
+
+
+# The 128-query kernel, which needs many heads: the requant extremes and the row-maximum wrap of
+# the tests above, and head dims above 64, where it runs over few keys (head_dim 64 with 560 heads of
+# 70 queries, 128 and 96 with 512 heads of 128).
+@pytest.mark.parametrize("B,Tq,Tk,D", [(280, 70, 150, 64), (256, 128, 128, 128), (256, 128, 70, 96)])
+@pytest.mark.parametrize("qs", [0, 1, 9, 14, 20, 27, 28, 29, 30, 31])
+def test_attention_prefill_extremes_many_heads(iw, oracle, gpu, B, Tq, Tk, D, qs):
+    H = 2
+    r = gen.rng(2000 + 31 * D + qs)
+    q = np.where(r.random((1, H, Tq, D)) < 0.5, -128, 127).astype(np.int8)
+    k = np.where(r.random((1, H, Tk, D)) < 0.5, -128, 127).astype(np.int8)
+    for t in range(0, Tk, 5):
+        k[:, :, t] = q[:, :, t % Tq]
+    for t in range(2, Tk, 7):
+        k[:, :, t] = np.where(q[:, :, (t + 3) % Tq] < 0, 127, -128)
+    v = gen.i8(r, (1, H, D, Tk))
+    qw, kw = q.copy(), k.copy()
+    qw[:, :, 5:40], kw[:, :, 1::3] = 127, -128  # rows that saturate beside rows that do not
+    for qm, qq, kk in ((0, q, k), (1, q, k), (255, q, k), (255, qw, kw)):
+        _print_case("attention prefill extremes, many heads", B, H, Tq, Tk, D, f"qs={qs} qm={qm}")
+        exp = oracle.attention(qq, kk, v, None, qm, qs, 8, 200, 6)
+        got = _fused(iw, *_copies(B, qq, kk, v), None, qm, qs, 8, 200, 6, decode=False)
+        assert np.array_equal(got, np.tile(exp, (B, 1, 1))), (qs, qm)
+
+
+# Either side of the lines between the kernels and their forms, at the number of heads where they
+# lie: two tiles per head with and without a padded chunk, pairs of tiles beyond two blocks per
+# CU, short and long keys, several full 64-key chunks with a ragged one and more tiles than the
+# 128-query kernel has blocks, head dims 32, 48 and above 64, held chunks for few and many blocks.
+@pytest.mark.parametrize("B,H,Tq,Tk,D", [
+    (104, 5, 40, 64, 64), (104, 5, 40, 65, 64), (104, 5, 33, 448, 48), (161, 5, 64, 800, 64), (161, 5, 64, 700, 64),
+    (60, 5, 65, 200, 64), (60, 5, 70, 1000, 64), (52, 5, 97, 330, 64), (220, 5, 70, 330, 64), (130, 10, 65, 40, 64),
+    (104, 5, 60, 64, 32), (208, 5, 60, 70, 32), (54, 10, 97, 300, 32), (80, 5, 128, 100, 96), (80, 5, 100, 64, 80),
+    (64, 8, 256, 256, 128), (80, 5, 128, 90, 112), (40, 5, 128, 128, 96), (52, 5, 65, 1000, 96), (40, 5, 12, 1201, 64),
+    (104, 5, 12, 700, 64), (104, 5, 12, 1250, 64), (36, 4, 66, 448, 64), (64, 4, 33, 1201, 64)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_prefill_kernel_choice(iw, oracle, gpu, B, H, Tq, Tk, D, masked):
+    _print_case("attention prefill kernel choice", B, H, Tq, Tk, D, masked)
+    q, k, v, qm, qs, f, am, as_ = gen.attn_case(B + Tq + 3 * Tk + D, 1, H, Tq, Tk, D)
+    mask = None
+    if masked:
+        mask = gen.rng(Tq).random((Tq, Tk)) < 0.3
+        mask[Tq // 3] = True
+    exp = oracle.attention(q, k, v, mask, qm, qs, f, am, as_)
+    got = _fused(iw, *_copies(B, q, k, v), mask, qm, qs, f, am, as_, decode=False)
+    assert np.array_equal(got, np.tile(exp, (B, 1, 1)))
+
+
 def test_argmax_rows(iw, gpu):
     r = gen.rng(9)
     x = gen.i8(r, (7, 51865))
