@@ -594,9 +594,12 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 //      lanes walk a row's 16-byte chunks, so each wave load reads 1 KB of one
 //      row; the per-lane partial sums are reduced once per row.
 constexpr int DC_MAX_TK = 4096;
-// Up to one block per CU 16 waves share a (batch, head), with every key load of
-// a 1500-key cache in flight; else 4. Head dim 96, us: 4 blocks 20.2 -> 13.4, 256
-// blocks 28.8 -> 25.1.
+// Up to one block per CU 16 waves share a (batch, head); else 4. 1024 threads leave a lane 128
+// registers, which hold a wave's first V^T chunk sets (two at head dim 96, one at 128) and eight
+// key loads; with more of either the compiler spills and every size is slower. us over 1500 keys
+// with four waves, with 16 that spill (12 key loads, two sets) and with these: head dim 96
+// 17.7 / 12.7 / 10.6 (4 blocks), 28.2 / 24.9 / 20.6 (256); head dim 128 19.0 / 17.4 / 10.9, 32.2 / 35.7 /
+// 24.6. Over 300 keys 8.6 / 10.3 / 7.7 and 9.6 / 14.3 / 8.2 (4 blocks).
 constexpr int64_t kManyWavesBlocks = 256;
 
 // NWV: waves per (batch, head).
@@ -606,7 +609,7 @@ __global__ __launch_bounds__(64 * NWV) void attn_decode_cache_kernel(AttnArgs a,
   constexpr int LPK = CPK <= 4 ? 4 : 8;            // lanes per key
   constexpr int KPW = 64 / LPK;                    // keys per wave load
   constexpr int RPW = D / NWV;                     // V^T rows per wave
-  constexpr int UK = NWV == 4 ? 4 : 12;            // key loads in flight per lane
+  constexpr int UK = NWV == 4 ? 4 : D == 64 ? 12 : 8;  // key loads in flight per lane
   constexpr int NT = 64 * NWV;
   static_assert(D % NWV == 0, "whole V^T rows per wave");
   __shared__ int32_t sS[DC_MAX_TK];
@@ -1668,7 +1671,7 @@ int launch_attn_decode_cache(const AttnArgs &a, const int32_t *pos, hipStream_t 
 #define IW_DC(D_, P_)                                                                                    \
   do {                                                                                                   \
     if (few)                                                                                             \
-      hipLaunchKernelGGL((attn_decode_cache_kernel<D_, 2, 16>), grid, dim3(1024), 0, s, a, pos);         \
+      hipLaunchKernelGGL((attn_decode_cache_kernel<D_, D_ == 128 ? 1 : 2, 16>), grid, dim3(1024), 0, s, a, pos); \
     else                                                                                                 \
       hipLaunchKernelGGL((attn_decode_cache_kernel<D_, P_, 4>), grid, dim3(256), 0, s, a, pos);          \
   } while (0)

@@ -80,17 +80,27 @@ def test_frag_bytes(iw):
     assert v("iw_frag_bytes", 1, 5121) == 0 and v("iw_frag_bytes", -1, 4) == 0
 
 
-def test_lds_loads_keep_their_wait_state(lib, tmp_path):
+LLVM = Path("/opt/rocm/llvm/bin")
+
+
+@pytest.fixture(scope="module")
+def code_objects(lib, tmp_path_factory):
+    """The gfx950 code objects of the built library."""
+    if not (LLVM / "llvm-objdump").exists():
+        pytest.skip("no llvm-objdump")
+    d = tmp_path_factory.mktemp("code")
+    shutil.copy(lib._name, d / "lib.so")
+    subprocess.run([LLVM / "llvm-objdump", "--offloading", "lib.so"], cwd=d, check=True, capture_output=True)
+    return sorted(d.glob("*gfx950*"))
+
+
+def test_lds_loads_keep_their_wait_state(code_objects):
     """A load into LDS takes its address from M0 and needs one wait state after a write of it. The
     compiler inserts none within inline assembly, so the built kernels are looked through."""
-    objdump = Path("/opt/rocm/llvm/bin/llvm-objdump")
-    if not objdump.exists():
-        pytest.skip("no llvm-objdump")
-    shutil.copy(lib._name, tmp_path / "lib.so")
-    subprocess.run([objdump, "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
     loads, bad = 0, []
-    for code in tmp_path.glob("*gfx950*"):
-        out = subprocess.run([objdump, "-d", "--no-show-raw-insn", code], check=True, capture_output=True, text=True)
+    for code in code_objects:
+        out = subprocess.run([LLVM / "llvm-objdump", "-d", "--no-show-raw-insn", code], check=True,
+                             capture_output=True, text=True)
         before = ""
         for line in out.stdout.splitlines():
             op = line.split("//")[0].strip()
@@ -100,3 +110,13 @@ def test_lds_loads_keep_their_wait_state(lib, tmp_path):
                     bad.append(op)
             before = op
     assert loads > 0 and not bad
+
+
+def test_decode_cache_attention_keeps_its_loads_in_registers(code_objects):
+    """A spilled operand load waits for its data before the next one is issued."""
+    spills = {}
+    for code in code_objects:
+        out = subprocess.run([LLVM / "llvm-readelf", "--notes", code], check=True, capture_output=True, text=True)
+        for m in re.finditer(r"\.name: +(\S*attn_decode_cache_kernel\S*).*?\.vgpr_spill_count: (\d+)", out.stdout, re.S):
+            spills[m[1]] = int(m[2])
+    assert len(spills) >= 7 and not any(spills.values()), spills

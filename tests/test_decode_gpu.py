@@ -427,6 +427,14 @@ def test_attention_decode_cross_lnq_block_counts(iw, oracle, gpu, B, H, Tk):
     test_attention_decode_cross_lnq(iw, oracle, gpu, B, H, Tk, True, True)
 
 
+# Head dims 96 and 128 on 16 waves: keys within and past the V^T chunk sets that a wave loads first.
+@pytest.mark.parametrize("B,H", [(1, 3), (16, 16)])
+@pytest.mark.parametrize("D,Tk", [(96, 1), (96, 129), (96, 2048), (96, 2049), (128, 15), (128, 1024), (128, 1025),
+                                  (128, 4096)])
+def test_attention_decode_cache_wide_heads(iw, oracle, gpu, B, H, D, Tk):
+    test_attention_decode_cache(iw, oracle, gpu, B, H, D, Tk, Tk, 1, "vt")
+
+
 # Two to four blocks per CU take eight waves per block: the edges of that range and of
 # the 256-key chunks.
 @pytest.mark.parametrize("B,H,Tk", [(33, 8, 1), (65, 16, 255), (86, 12, 257), (64, 16, 1500), (52, 20, 513),
