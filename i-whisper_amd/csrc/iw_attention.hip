@@ -803,23 +803,34 @@ __global__ __launch_bounds__(64 * NWV) void attn_decode_cache_kernel(AttnArgs a,
 #ifndef IW_DS_CH
 #define IW_DS_CH 128
 #endif
-// Grids of at most one block per CU take 16 waves per (batch, head), 256-key
-// chunks and four slots (64 KB): there a block has its CU to itself and what
-// bounds it is the chain of its own steps, four times shorter per wave (a
-// deeper ring for the four waves changes nothing). us per launch over 1500
-// HBM-cold keys: 20 blocks 11.0 -> 8.2, 256 blocks 14.4 -> 12.2; three queries
-// 24.6 -> 16.1; with LayerNorm and query 14.8 -> 11.8 and 17.3 -> 15.2. From two
-// blocks per CU the chains of several small blocks overlap and the forms
-// tie (324 blocks: 17.1 and 17.8).
+// Up to one block per CU 16 waves per (batch, head), 256-key chunks and four slots (64 KB): there a
+// block has its CU to itself and what bounds it is the chain of its own steps, four times shorter
+// per wave (a deeper ring for the four waves changes nothing). us per launch over 1500 HBM-cold keys:
+// 20 blocks 11.0 -> 8.2, 256 blocks 14.4 -> 12.2; three queries 24.6 -> 16.1; with LayerNorm and query
+// 14.8 -> 11.8 and 17.3 -> 15.2. A few chunks are no chain, and then the larger barriers and sums
+// cost more than they save; the fuller the chip, the later the wide form pays: stream_many_waves,
+// lnq_waves. us with four and with 16 waves over 300 / 600 / 1000 keys: two queries, 20 blocks
+// 7.3 / 7.7, 9.4 / 8.6, 12.2 / 9.5; the fused form, 20 blocks 8.0 / 8.4, 9.6 / 9.2, 11.7 / 10.1, 256 blocks
+// 8.5 / 9.2, 10.1 / 10.6, 12.6 / 11.8.
 constexpr int DM_NW = 16, DM_NR = 4, DM_CH = 256;
-constexpr int64_t kManyWavesMaxBlocks = 256;
 // The fused cross-attention from there to four blocks per CU: eight waves with the
 // same chunks and slots (two blocks per CU). us per token step with four and eight
 // waves: 264 / 324 / 504 blocks of 768 channels 725 -> 707, 737 -> 714, 753 -> 725; 500 / 800
 // of 1280 2160 -> 2081, 2547 -> 2491; 1024 of 1024 1957 -> 1912; 2560 4440 and 4439 (128-key chunks
-// or three slots are 0.2 to 6 % slower at all of them).
+// or three slots are 0.2 to 6 % slower at all of them). us per launch over 300 / 800 / 1500
+// keys: 324 blocks 10.2 / 10.8, 13.8 / 13.6, 20.5 / 18.3, 1024 blocks 14.3 / 19.6, 25.5 / 29.3, 40.0 / 39.8.
 constexpr int DH_NW = 8;
-constexpr int64_t kHalfWavesMaxBlocks = 1024;
+constexpr int64_t kStreamCus = 256;
+
+bool stream_many_waves(int64_t blocks, int keys, bool several_queries) {
+  if (blocks > kStreamCus) return false;
+  return keys > (several_queries || blocks <= 3 * kStreamCus / 4 ? 384 : 640);
+}
+
+int lnq_waves(int64_t blocks, int keys) {
+  if (blocks <= kStreamCus) return keys > 384 + 3 * blocks / 2 ? DM_NW : 4;
+  return blocks <= 4 * kStreamCus && keys > (blocks <= 2 * kStreamCus ? 768 : 1400) ? DH_NW : 4;
+}
 
 // the self-attention instance (at most 512 keys) has its own ring shape
 #ifndef IW_DSS_NR
@@ -1596,10 +1607,11 @@ int launch_attn_decode_cross_lnq(const AttnArgs &a, const LnQueryArgs &lq, hipSt
       lq.hidden > 1280 || lq.kp > 1280 || lq.code < 0)
     return fail("the fused cross-attention takes head_dim 64, V transposed, at most 2048 keys and 1280 channels");
   const dim3 grid((unsigned)(a.B * a.H));
-  if (grid.x <= kManyWavesMaxBlocks)
+  const int nw = lnq_waves(grid.x, a.Tk);
+  if (nw == DM_NW)
     hipLaunchKernelGGL((attn_decode_cross_lnq_kernel<DM_NR, DM_CH, DM_NW>), grid, dim3(64 * DM_NW), 0, s,
                        a, lq);
-  else if (grid.x <= kHalfWavesMaxBlocks)
+  else if (nw == DH_NW)
     hipLaunchKernelGGL((attn_decode_cross_lnq_kernel<DM_NR, DM_CH, DH_NW>), grid, dim3(64 * DH_NW), 0, s,
                        a, lq);
   else
@@ -1626,9 +1638,9 @@ int launch_attn_decode_cache(const AttnArgs &a, const int32_t *pos, hipStream_t 
   if (a.max_tk <= 512)                                                                                         \
     hipLaunchKernelGGL((attn_decode_stream_kernel<512, IW_DSS_NR, IW_DSS_CH, IW_DSS_NW, VQ_>), grid,            \
                        dim3(64 * IW_DSS_NW), 0, s, a, pos);                                                    \
-  else if (a.max_tk <= 2048 && grid.x <= kManyWavesMaxBlocks)                                                  \
-    hipLaunchKernelGGL((attn_decode_stream_kernel<2048, DM_NR, DM_CH, DM_NW, VQ_>), grid,              \
-                       dim3(64 * DM_NW), 0, s, a, pos);                                                     \
+  else if (a.max_tk <= 2048 && many)                                                                           \
+    hipLaunchKernelGGL((attn_decode_stream_kernel<2048, DM_NR, DM_CH, DM_NW, VQ_>), grid, dim3(64 * DM_NW), 0, s, a, \
+                       pos);                                                                                   \
   else if (a.max_tk <= 2048)                                                                                   \
     hipLaunchKernelGGL((attn_decode_stream_kernel<2048, IW_DS_NR, IW_DS_CH, 4, VQ_>), grid, dim3(256), 0, s, a, \
                        pos);                                                                                   \
@@ -1658,6 +1670,9 @@ int launch_attn_decode_cache(const AttnArgs &a, const int32_t *pos, hipStream_t 
                            tpf, tstart);
       return check_launch("attn_decode_self_kernel");
     }
+    // with pos the number of keys is on the device, any up to max_tk: taken for half of it (a cache
+    // of 1500 keys, us with four and with 16 waves: 100 in use 3.6 / 4.7, all 10.9 / 8.0)
+    const bool many = stream_many_waves(grid.x, pos ? a.max_tk / 2 : a.Tk, false);
     if (vq) {
       IW_DS(true)
     } else {
@@ -1707,7 +1722,7 @@ int launch_attn_decode(const AttnArgs &a, hipStream_t s) {
     c.o_frag_kp = 0;
     const dim3 grid((unsigned)(a.B * a.H));
 #define IW_DQ(NQ_)                                                                                                 \
-  if (grid.x <= kManyWavesMaxBlocks)                                                                               \
+  if (stream_many_waves(grid.x, a.Tk, NQ_ > 1))                                                                    \
     hipLaunchKernelGGL((attn_decode_stream_kernel<2048, DM_NR, DM_CH, DM_NW, false, NQ_>), grid,           \
                        dim3(64 * DM_NW), 0, s, c, nullptr);                                                     \
   else                                                                                                             \

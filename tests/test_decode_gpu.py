@@ -441,3 +441,15 @@ def test_attention_decode_cache_wide_heads(iw, oracle, gpu, B, H, D, Tk):
                                     (43, 6, 2048), (13, 20, 1500)])
 def test_attention_decode_cross_lnq_eight_waves(iw, oracle, gpu, B, H, Tk):
     test_attention_decode_cross_lnq(iw, oracle, gpu, B, H, Tk, True, True)
+
+
+# The keys from which a block takes more waves, by blocks per CU: 16 up to one, eight up to four.
+@pytest.mark.parametrize("B,H,Tk", [(1, 6, 393), (1, 6, 394), (16, 16, 768), (16, 16, 769), (33, 8, 768), (33, 8, 769),
+                                    (64, 8, 769), (43, 12, 1400), (43, 12, 1401), (64, 16, 1401), (65, 16, 1401)])
+def test_attention_decode_cross_lnq_wave_lines(iw, oracle, gpu, B, H, Tk):
+    test_attention_decode_cross_lnq(iw, oracle, gpu, B, H, Tk, True, True)
+
+
+@pytest.mark.parametrize("B,H,Tk", [(16, 12, 512), (16, 12, 513), (16, 16, 640), (16, 16, 641), (2, 8, 2048)])
+def test_attention_decode_cache_wave_lines(iw, oracle, gpu, B, H, Tk):
+    test_attention_decode_cache(iw, oracle, gpu, B, H, 64, Tk, Tk, 1, "vt")

@@ -447,6 +447,13 @@ def test_attention_strided_mask(iw, oracle, gpu, B, H, Tq, Tk, D):
         iw._lib.call("iw_attention_strided_mask", *args, Tk - 1, *tail)
 
 
+@pytest.mark.parametrize("B,H,Tq,Tk", [(1, 5, 1, 384), (1, 5, 1, 385), (16, 16, 1, 640), (16, 16, 1, 641), (1, 5, 2, 384),
+                                       (1, 5, 2, 385), (16, 16, 4, 385), (16, 16, 8, 400), (17, 16, 1, 1500)])
+def test_attention_decode_wave_lines(iw, oracle, gpu, B, H, Tq, Tk):
+    """The keys from which a block of the shared stream takes 16 waves, for one query and for several."""
+    test_attention_decode_fused(iw, oracle, gpu, B, H, Tq, Tk, 64, False)
+
+
 @pytest.mark.parametrize("decode", [False, True])
 def test_attention_fused_wrap_corner(iw, oracle, gpu, decode):
     """Scores saturating at +32767 wrap rmp1 and give P = 128 at x_sub = 0."""
