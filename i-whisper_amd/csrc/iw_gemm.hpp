@@ -226,7 +226,7 @@ int launch_frag_pack(const int8_t *src, int64_t rows, int64_t cols, int64_t ld, 
 constexpr int64_t kBigGemmMinRows = 8192;
 
 int gemm_dense(const GemmArgs &g, hipStream_t s);
-int gemm_big(const GemmArgs &g, hipStream_t s);
+int gemm_big(const GemmArgs &g, bool conv_cl, hipStream_t s);
 // Direct-to-LDS kernels (iw_gemm_dtl.hip): dense A, K % 128 == 0 (64 from
 // kBigGemmMinRows rows), N % 16 == 0, 16-byte aligned.
 bool gemm_dtl_eligible(const GemmArgs &g);

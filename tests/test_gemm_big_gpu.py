@@ -153,6 +153,38 @@ def test_conv1d_channels_last_big(iw, oracle, gpu, B, Cin, Tin, Cout, stride):
     assert np.array_equal(host(out16), exp16)
 
 
+# What the direct-to-LDS tiles do not take, on both sides of 8192 rows: an output and a positional
+# table at odd addresses, and a ragged number of channels with several column tiles.
+@pytest.mark.parametrize("B,Cin,Tin,Cout,stride,off", [(1, 48, 3000, 144, 2, 1), (6, 48, 3000, 144, 2, 1),
+                                                       (3, 32, 3000, 296, 1, 0), (2, 32, 4097, 136, 1, 1)])
+def test_conv1d_channels_last_unaligned(iw, oracle, gpu, B, Cin, Tin, Cout, stride, off):
+    print("case: conv1d_cl unaligned", B, Cin, Tin, Cout, stride, off, flush=True)
+    r = gen.rng(B * Cin + Tin + Cout)
+    x = gen.i8(r, (B, Cin, Tin))
+    w = gen.i8(r, (Cout, Cin * 3), -60, 60)
+    bias = r.integers(-2**16, 2**16, size=Cout).astype(np.int32)
+    mult, shift = int(r.integers(2**29, 2**31)), 9
+    gp = gen.gelu_params(r, Cout, False, True)
+    g = oracle.gelu(np.ascontiguousarray(oracle.conv1d(x, w, bias, mult, shift, stride, 1).transpose(0, 2, 1)), *gp)
+    tout = g.shape[1]
+    pe = gen.i8(r, (tout, Cout))
+    pm, ps = r.integers(1, 65536, size=Cout).astype(np.uint16), r.integers(-1, 12, size=Cout).astype(np.int8)
+    exp16 = oracle.add_requant15(g, pe, pm, ps)
+    ts = [T(np.ascontiguousarray(x.transpose(0, 2, 1))), T(_kc(w, Cin, 3)), T(bias)]
+    gt, pms = [T(a) for a in gp], [T(pm), T(ps)]
+    peb = torch.zeros(tout * Cout + off, dtype=torch.int8, device="cuda")
+    peb[off:] = T(pe).view(-1)
+    for pos, exp, dtype in ((False, g, torch.int8), (True, exp16, torch.int16)):
+        buf = torch.zeros(exp.size + 2 * off, dtype=dtype, device="cuda")
+        out = buf[off:off + exp.size]
+        iw._lib.call("iw_conv1d_cl", *(t.data_ptr() for t in ts), mult, shift, *(t.data_ptr() for t in gt), 1, Cout,
+                     peb[off:].data_ptr() if pos else None, *(t.data_ptr() if pos else None for t in pms),
+                     Cout if pos else 0, Cout if pos else 0, out.data_ptr(), B, Cin, Tin, Cout, 3, stride, 1, True,
+                     stream())
+        assert np.array_equal(host(out).reshape(exp.shape), exp)
+        assert not off or (int(buf[0]) == 0 and int(buf[-1]) == 0)
+
+
 # Convolutions over the direct-to-LDS tiles: one position, rows without any tap
 # inside the input, K of no whole stage, ragged rows and columns, sequences that
 # end inside a tile, each tile size, GeLU as a table and per channel.
