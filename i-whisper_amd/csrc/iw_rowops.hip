@@ -1259,10 +1259,12 @@ int launch_quantize_mel(const float *mel, float alpha, int8_t *out, int64_t b, i
   return check_launch("quantize_mel_kernel");
 }
 
-// 128 x 128 tiles from here on, where they fill the chip: us with 64 x 64 and 128 x 128
-// tiles, 128 x 1500 x 1280 171 / 148, 64 x 1500 x 1024 63.5 / 50.0, 16 x 1500 x 512 (768 tiles)
-// 8.8 / 6.5, 5 x 1500 x 1024 (480) 6.2 / 5.2, 3 x 677 x 768 (108) 3.1 / 3.5.
-constexpr int64_t kTransposeTiles128 = 400;
+// 128 x 128 tiles from here on, where they fill the chip and the positions more than half a
+// tile (a decoder prompt's do not): us with 64 x 64 and 128 x 128 tiles, 128 x 1500 x 1280
+// 171 / 148, 64 x 1500 x 1024 63.5 / 50.0, 16 x 1500 x 512 (768 tiles) 8.8 / 6.5, 5 x 1500 x 1024 (480)
+// 6.2 / 5.2, 3 x 677 x 768 (108) 3.1 / 3.5; 128 x 72 x 1280 15.8 / 11.8, 128 x 64 x 1280 6.5 / 6.0,
+// 128 x 48 x 1280 5.2 / 5.6, 128 x 3 x 1280 3.8 / 5.4.
+constexpr int64_t kTransposeTiles128 = 400, kTransposePositions128 = 64;
 
 int launch_transpose_heads(const int8_t *src, int64_t src_sb, int64_t src_st, int8_t *dst,
                            int64_t dst_sb, int64_t dst_sh, int64_t dst_sd, int64_t dst_sq, int64_t t_off,
@@ -1274,7 +1276,7 @@ int launch_transpose_heads(const int8_t *src, int64_t src_sb, int64_t src_st, in
                        (uintptr_t)t_off | (uintptr_t)(H * D);
   if (dst_sq == 4 && (al & 15) == 0 && H * D <= 0x7fffffff) {
     const int64_t tt = (T + TH_T - 1) / TH_T, tc = (H * D + TH_C - 1) / TH_C, tiles = tt * tc * B;
-    if (tiles >= kTransposeTiles128 && tiles <= 0x3fffffff) {
+    if (T >= kTransposePositions128 && tiles >= kTransposeTiles128 && tiles <= 0x3fffffff) {
       const unsigned per_xcd = (unsigned)((tiles + 7) / 8);
       hipLaunchKernelGGL(transpose_heads128_kernel, dim3(8 * per_xcd), dim3(256), 0, s, src, src_sb, src_st, dst, dst_sb,
                          dst_sh, dst_sd, t_off, T, H, D, (unsigned)tt, (unsigned)tc, (unsigned)tiles, per_xcd);

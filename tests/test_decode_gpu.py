@@ -210,9 +210,11 @@ def test_transpose_heads(iw, gpu, B, T, H, D, t_off, layout):
 
 
 @pytest.mark.parametrize("B,T,H,D,t_off", [(60, 333, 7, 48, 16), (5, 1500, 16, 64, 0), (200, 130, 2, 64, 0),
-                                           (401, 1, 1, 16, 0)])
+                                           (401, 1, 1, 16, 0), (130, 63, 7, 64, 0), (130, 64, 7, 64, 16),
+                                           (130, 65, 7, 64, 0)])
 def test_transpose_heads_many(iw, gpu, B, T, H, D, t_off):
-    """Enough 128 x 128 tiles for the large form: ragged positions and columns."""
+    """Enough 128 x 128 tiles for the large form: ragged positions and columns, and the
+    positions from which it is taken."""
     test_transpose_heads(iw, gpu, B, T, H, D, t_off, "vt")
 
 
