@@ -19,15 +19,17 @@ constexpr int64_t kCus = 256;
 // them per product: 64 x 64 tiles take 0.26 us per stage for 1/16 of the work
 // that 256 x 256 tiles do in 1.8 us; but 1500 rows of a width of 1280 are only
 // 30 tiles of 256 x 256 and 480 of 64 x 64. `fixed` is the launch with its
-// first loads, `tail` the requantization and stores of a tile. Fitted to 360
-// launches (M = 130 .. 48000, the QKV, out-projection, FC1 and FC2 shapes of
-// widths 384 .. 1280), where the tile that it picks is 0.1 % slower in the
-// geometric mean than the best of the four, and 5 % at most.
+// first loads, `tail` the requantization and stores of a tile, `lone` the
+// factor of a launch that is over in one round. Over 976 launches (M = 129 .. 96000,
+// the QKV, out-projection, FC1 and FC2 shapes of widths 384 .. 1280 and a few others,
+// with and without GeLU), the tile that it picks is 0.4 % slower in the geometric
+// mean than the best of the four, and 22 % at most. Without `lone`, 9000 x 1536 x 384
+// (216 tiles of 256 x 256) ran 17.4 us on 128 x 128, 15.7 on 256 x 256.
 struct TileCost {
   int64_t bm, bn, per_cu;
-  double shared, alone, fixed, tail;
+  double shared, alone, fixed, tail, lone = 1;
 };
-constexpr TileCost kCost256{Tile256::BM, Tile256::BN, 1, 1.8, 1.75, 7.0, 2.56};
+constexpr TileCost kCost256{Tile256::BM, Tile256::BN, 1, 1.8, 1.75, 7.0, 2.56, 0.92};
 constexpr TileCost kCost128{Tile128::BM, Tile128::BN, 2, 0.53, 0.964, 4.67, 0.745};
 constexpr TileCost kCost64x128{Tile64x128::BM, Tile64x128::BN, 3, 0.361, 0.571, 3.5, 0.6};
 constexpr TileCost kCost64{Tile64::BM, Tile64::BN, 2, 0.263, 0.285, 3.96, 0.33};
@@ -39,7 +41,7 @@ double tile_us(const TileCost &c, const GemmArgs &g) {
   const int64_t rounds = tiles / (kCus * c.per_cu), rest = tiles % (kCus * c.per_cu);
   double us = c.fixed + (double)(rounds * c.per_cu) * one;
   if (rest) us += std::max(c.alone * stages + c.tail, (double)((rest + kCus - 1) / kCus) * one);
-  return us;
+  return tiles <= kCus * c.per_cu ? c.lone * us : us;
 }
 
 }  // namespace
@@ -79,7 +81,11 @@ bool gemm_dtl_conv_eligible(const GemmArgs &g) {
 int gemm_dtl(const GemmArgs &g, hipStream_t s) {
   if (g.K % 128 != 0 && g.conv_cin == 0) return gemm_dtl_tile<Tile256>(g, s);  // the others' stages are 128 bytes of K
   const double us256 = tile_us(kCost256, g), us128 = tile_us(kCost128, g);
-  const double us64x128 = tile_us(kCost64x128, g), us64 = tile_us(kCost64, g);
+  // the columns' own GeLU parameters take the LDS of the third 64 x 128 block (1500 x 4096 x 1024:
+  // 21.1 us there, 17.9 on 128 x 128)
+  TileCost c64x128 = kCost64x128;
+  if (g.lut && (g.luti_pc || g.luto_pc)) c64x128.per_cu = 2;
+  const double us64x128 = tile_us(c64x128, g), us64 = tile_us(kCost64, g);
   const double best = std::min(std::min(us256, us128), std::min(us64x128, us64));
   if (best == us256) return gemm_dtl_tile<Tile256>(g, s);
   if (best == us128) return gemm_dtl_tile<Tile128>(g, s);

@@ -628,7 +628,7 @@ int gemm_dtl_tile(const GemmArgs &g, hipStream_t s) {
 // The tiles in use, each instantiated in a translation unit of its own.
 using Tile256 = Tile<2, 4, 4, 2, 64, 4, 2, false>;   // 256 x 256, one block per CU
 using Tile128 = Tile<2, 2, 2, 2, 128, 2, 2, true>;   // 128 x 128, two
-using Tile64x128 = Tile<2, 2, 1, 2, 128, 2, 3, true>;  // 64 x 128, three
+using Tile64x128 = Tile<2, 2, 1, 2, 128, 2, 3, true>;  // 64 x 128, three (two with per-column GeLU)
 using Tile64 = Tile<2, 2, 1, 1, 128, 4, 2, true>;    // 64 x 64, two
 extern template int gemm_dtl_tile<Tile256>(const GemmArgs &, hipStream_t);
 extern template int gemm_dtl_tile<Tile128>(const GemmArgs &, hipStream_t);
