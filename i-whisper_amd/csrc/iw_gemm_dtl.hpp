@@ -589,7 +589,7 @@ int launch_dtl(const GemmArgs &g, hipStream_t s) {
   if (tiles == 0) return 0;
   const int per_xcd = (int)((tiles + XCDS - 1) / XCDS);
   const dim3 grid((unsigned)(per_xcd * XCDS)), block(T::NT);
-  if constexpr (!CONV) {
+  if constexpr (EPI != EPI_S8) {  // per-tensor outputs (convolutions, the classifier) have no zero points
     if (g.wz) {
       hipLaunchKernelGGL((gemm_dtl_kernel<EPI, GELU, true, GT, false, false, T>), grid, block, 0, s, g, (int)tn,
                          (int)tiles, per_xcd);
@@ -619,7 +619,7 @@ int gemm_dtl_tile(const GemmArgs &g, hipStream_t s) {
     case EPI_L32: return launch_dtl<EPI_L32, false, false, T>(g, s);
     case EPI_L32RES: return launch_dtl<EPI_L32RES, false, false, T>(g, s);
     case EPI_S8:
-      if (gelu) return launch_dtl<EPI_S8, true, false, T>(g, s);
+      if (gelu || g.wz) return fail("the dense per-tensor epilogue (the classifier) has no GeLU and no zero points");
       return launch_dtl<EPI_S8, false, false, T>(g, s);
     default: return fail("unknown GEMM epilogue");
   }
