@@ -220,7 +220,7 @@ def test_layernorm32(iw, oracle, gpu, hidden, rows, spread):
 def test_layernorm32_full_int16_range(iw, oracle, gpu, hidden, rows):
     """Rows whose deviations from the mean exceed 46340, where d^2 wraps in int32
     (the kernels' per-element form), next to ordinary rows in the same launch:
-    row-per-block launches (<= 2048 rows) and one persistent-wave launch."""
+    row-per-block launches (<= 256 rows) and one persistent-wave launch."""
     _print_case("layernorm32 full int16 range", hidden, rows)
     x, g, b, lm, ls, om, os_ = gen.ln_case(hidden + rows + 1, rows, hidden, 3000)
     r = gen.rng(rows)
@@ -236,6 +236,24 @@ def test_layernorm32_full_int16_range(iw, oracle, gpu, hidden, rows):
         T(x), T(g), T(b), torch.tensor([lm], dtype=torch.uint8), torch.tensor([ls], dtype=torch.int8),
         torch.tensor([om], dtype=torch.uint32), torch.tensor([os_], dtype=torch.int8))
     assert np.array_equal(host(got), oracle.layernorm32(x, g, b, lm, ls, om, os_))
+
+
+@pytest.mark.parametrize("hidden", [384, 512, 768, 1024, 1280])
+@pytest.mark.parametrize("rows", [256, 257, 3001])
+@pytest.mark.parametrize("out_m", [0x40000001, 0x7fffffff, 0x80000000, 0xc0000001])
+def test_layernorm32_wave_rows(iw, oracle, gpu, hidden, rows, out_m):
+    """Every width on wave rows (and the last row-per-block launch), the output multiplier on both
+    sides of 2^31, rows whose squares wrap among ordinary ones and a row that is constant."""
+    _print_case("layernorm32 wave rows", hidden, rows, out_m)
+    x, g, b, lm, ls, _, os_ = gen.ln_case(hidden + rows, rows, hidden, 3000)
+    x[0], x[0, 5] = 32767, -32768
+    x[1], x[1, -1] = -32768, 32767
+    x[rows // 2] = gen.rng(rows).integers(-32768, 32768, size=hidden)
+    x[rows - 1] = 77
+    got = iw.kernels.layernorm32_hip(
+        T(x), T(g), T(b), torch.tensor([lm], dtype=torch.uint8), torch.tensor([ls], dtype=torch.int8),
+        torch.tensor([out_m], dtype=torch.uint32), torch.tensor([os_], dtype=torch.int8))
+    assert np.array_equal(host(got), oracle.layernorm32(x, g, b, lm, ls, out_m, os_))
 
 
 @pytest.mark.parametrize("rows", [3, 5000])
@@ -472,7 +490,8 @@ def test_attention_fused_wrap_corner(iw, oracle, gpu, decode):
 def test_attention_prefill_requant_extremes(iw, oracle, gpu, D, qs):
     """Scores at the int8 extremes (|QK^T| up to 128 * 128 * D) against every
     requant shift and the multipliers 0, 1 and 255, over key chunks that are
-    full (64 keys) and a ragged last one: keys aligned with the query (largest
+    full (32 keys: at this size 32-query tiles; test_attention_prefill_extremes_many_heads
+    has the 128-query kernel's 64) and a ragged last one: keys aligned with the query (largest
     scores, saturating the int16 row maximum for small shifts), anti-aligned
     (most negative) and random signs."""
     B, H, Tq, Tk = 1, 2, 70, 150
@@ -492,7 +511,7 @@ def test_attention_prefill_requant_extremes(iw, oracle, gpu, D, qs):
 
 
 def test_attention_prefill_wrap_in_full_chunks(iw, oracle, gpu):
-    """The row-maximum wrap (P = 128 at x_sub = 0) inside full 64-key chunks:
+    """The row-maximum wrap (P = 128 at x_sub = 0) inside full key chunks (32 keys at this size):
     every query row saturates at +32767 while a third of the keys sit at
     -32768."""
     B, H, Tq, Tk, D = 1, 2, 33, 200, 64

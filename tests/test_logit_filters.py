@@ -204,6 +204,47 @@ def test_filtered_greedy_step_matches_oracle(iw, gpu, rules):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("V,tb,eot", [(7, 5, 4), (16, 12, 11), (33, 30, 28), (1100, 900, 880)])
+@pytest.mark.parametrize("all_text", [False, True])
+def test_filtered_greedy_step_short_rows(iw, gpu, V, tb, eot, all_text):
+    """Vocabularies below and around one 16-byte piece, rows that start at every address mod 16, and
+    every text token suppressed (the sums are then over timestamps alone, or over nothing)."""
+    print("filtered greedy, short rows:", V, tb, eot, all_text, flush=True)
+    rng = np.random.default_rng(V + all_text)
+    spec = FilterSpec(sample_begin=1, eot=eot, suppress_tokens=list(range(tb)) if all_text else [1],
+                      timestamp_begin=tb, no_timestamps=eot - 1, max_initial_timestamp_index=1)
+    B, ld, hist_cols, scale = 16, (V + 15) // 16 * 16 + 1, 12, 0.0917
+    mask = torch.from_numpy(bitmask(spec.suppress_tokens + [spec.no_timestamps], V)).cuda()
+    prompt = np.full((B, 1), 2, np.int64)
+    prev0 = torch.from_numpy(prompt[:, 0].copy()).cuda()
+    for st in (0, 1, 2, 5):
+        q = random_case(rng, B, V, tb, eot, B // 2)
+        hist = np.array([history_for(rng, st, V, tb, eot) for _ in range(B)], np.int64).reshape(B, st)
+        toks = np.concatenate([prompt, hist], 1)
+        f32 = q.astype(np.float32) * np.float32(scale)
+        keep = timestamp_margin(f32, toks, spec) > 1e-3
+        want = greedy_next(f32, toks, spec)
+        buf = torch.full((B, ld), 127, dtype=torch.int8, device="cuda")
+        buf[:, :V] = torch.from_numpy(q).cuda()
+        ht = torch.zeros((B, hist_cols), dtype=torch.int64, device="cuda")
+        ht[:, :st] = torch.from_numpy(hist).cuda()
+        nxt = torch.empty(B, dtype=torch.int64, device="cuda")
+        step, pos = (torch.tensor([v], dtype=torch.int32, device="cuda") for v in (st, 1 + st))
+        slp0 = rng.normal(-5, 2, B).astype(np.float32)
+        slp = torch.from_numpy(slp0.copy()).cuda()
+        cnt = torch.zeros(hist_cols, dtype=torch.int32, device="cuda")
+        iw._lib.call("iw_greedy_advance_filtered", buf.data_ptr(), B, V, ld, nxt.data_ptr(), ht.data_ptr(), hist_cols,
+                     hist_cols, step.data_ptr(), pos.data_ptr(), 1, mask.data_ptr(), None, prev0.data_ptr(), eot, tb,
+                     1, scale, slp.data_ptr(), cnt.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        got, g_slp = nxt.cpu().numpy(), slp.cpu().numpy()
+        assert np.array_equal(got[keep], want[keep]), st
+        _, w_slp, _ = greedy_update(apply_filters(f32, toks, spec), toks, eot, slp0)
+        assert np.array_equal(np.isnan(g_slp[keep]), np.isnan(w_slp[keep]))
+        fin = keep & ~np.isnan(w_slp)
+        assert np.allclose(g_slp[fin], w_slp[fin], rtol=1e-5, atol=1e-4), st
+
+
+@pytest.mark.gpu
 def test_greedy_decode_with_filters(iw, gpu):
     """End to end on the golden 1+1-layer model: every step's token is the
     filtered greedy choice over that step's int8 logits and the tokens so far,

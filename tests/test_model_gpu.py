@@ -146,6 +146,27 @@ def test_decoder_layers_read_the_mask_themselves(iw, small, n_tok):
     assert torch.equal(got, exp)
 
 
+@pytest.mark.parametrize("batch,n_tok", [(2, 5), (9, 20)])
+def test_decoder_float_logits_by_either_way(iw, small, batch, n_tok):
+    """The logits divided in one call (a one-element float32 alpha) and by classify and torch (alphas
+    of other shapes and types) are the same, below and above the decode kernel's 128 rows."""
+    dims, P, model, ref = small
+    dec = model.decoder
+    xa = T(ref.encoder(iw.synth.synthetic_mel(batch, dims.n_mels, 2 * dims.n_audio_ctx, seed=34)))
+    toks = T(gen.rng(n_tok).integers(0, dims.n_vocab, size=(batch, n_tok)).astype(np.int64))
+    keep = dec.act_logits_alpha
+    try:
+        with torch.no_grad():
+            one = dec(toks, xa)
+            for alpha in (keep.detach().reshape(()), keep.detach().reshape(1, 1, 1), keep.detach().expand(dims.n_vocab),
+                          keep.detach().double()):
+                dec.act_logits_alpha = torch.nn.Parameter(alpha.clone())
+                got = dec(toks, xa)
+                assert got.dtype == alpha.dtype and torch.equal(got.float(), one)
+    finally:
+        dec.act_logits_alpha = keep
+
+
 @pytest.mark.parametrize("batch,steps", [(1, 6), (3, 10)])
 def test_greedy_decode_runner(iw, small, batch, steps):
     dims, P, model, ref = small
