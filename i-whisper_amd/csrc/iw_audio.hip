@@ -115,8 +115,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 //   B[q][m][s] = W64^(m s) sum_j A_q[m + 8 j] W8^(j s)          lane 8 q + m
 //   X[q + 8 s + 64 t] = sum_m B[q][m][s] W8^(m t)               lane 8 s + q
 // (W_n = exp(-2 pi i / n), from a table computed in float64 on the host). The
-// LDS rows are laid out so that neither side of an exchange meets a bank
-// twice. Each mel bin then sums its filter's nonzero taps (sparse rows: first
+// LDS rows are laid out so that an exchange's lanes spread over the banks (the writes
+// of B alone meet seven of the 64 banks twice: 72 s + 9 m + q). Each mel bin then sums its
+// filter's nonzero taps (sparse rows: first
 // bin, tap count, offset into the weights), and the block writes [n_mels][64]
 // rows of log10 values plus its maximum. With 4 waves of 16 frames and nine
 // radix-2 steps in LDS this took 85.8 us for 30 s of audio at 80 mels; now 21.8.

@@ -588,9 +588,12 @@ __device__ __forceinline__ uint32_t range_bits16(int i0, int lo, int hi) {
 
 // A row is one block's, so the time is that of its chain: 1024 threads read the
 // row in 16-byte pieces twice, for the maxima and then for the sums of
-// exp((x - max) scale) from a 256-entry table in LDS (one expf per value
-// instead of one per logit). A pass of 256 threads, a byte and an expf at a
-// time, took 62.6 us per step for 27 rows of 51865 logits; this takes 12.
+// exp((x - max) scale) from a 256-entry table in LDS (one exponential per value,
+// in 64 bits and rounded, instead of an expf per logit). A pass of 256 threads, a byte
+// and an expf at a time, took 62.6 us per step for 27 rows of 51865 logits; this takes
+// 17.1 with the log-probability sums and 13.6 without them. A step's log-probability is off by
+// 1.5e-7 (rms; the pass of expf 2.7e-7); its sum over the steps by the rounding of the
+// 32-bit sum itself, about 1e-7 of it either way.
 constexpr int GF_NT = 1024, GF_NW = GF_NT / 64;
 
 __global__ __launch_bounds__(GF_NT) void greedy_filtered_kernel(const int8_t *__restrict__ x, int64_t cols,
