@@ -332,11 +332,8 @@ class MultiHeadAttention_int(_ScalarCache, nn.Module):
         Tk = k.shape[1]
         H = self.n_head
         D = C // H
-        attn_mask = None
-        if mask is not None:  # model_int.py:786-799
-            q_offset = Tk - Tq
-            assert q_offset >= 0
-            attn_mask = mask[q_offset:q_offset + Tq, :Tk]
+        q_offset = Tk - Tq
+        assert mask is None or q_offset >= 0
         s = self._scalars()
         out = torch.empty((B, Tq, C), dtype=torch.int8, device=q.device)
         if D % 16 == 0 and D <= 128 and Tk <= 4096:
@@ -350,15 +347,18 @@ class MultiHeadAttention_int(_ScalarCache, nn.Module):
             tp = vt.shape[-1]
             decode = Tq <= 8
             table = None if decode else self.shift_exp_table()
-            ld = Tk
-            if attn_mask is not None:  # read in place where its rows are whole bytes side by side
-                if attn_mask.element_size() != 1 or attn_mask.stride(1) != 1 or attn_mask.stride(0) < Tk:
-                    attn_mask = attn_mask.contiguous()
+            mp, ld = None, Tk
+            if mask is not None:  # model_int.py:786-799
+                if mask.dtype == torch.bool and mask.is_contiguous() and mask.dim() == 2 and min(mask.shape) >= Tk:
+                    # rows q_offset .. of the mask, read where they are
+                    ld = mask.shape[1]
+                    mp = mask.data_ptr() + q_offset * ld
                 else:
-                    ld = attn_mask.stride(0)
+                    mask = mask[q_offset:q_offset + Tq, :Tk].contiguous()
+                    mp = mask.data_ptr()
             _lib.call("iw_attention_strided_mask", q.data_ptr(), Tq * C, C, k.data_ptr(), Tk * C, D, C,
                       vt.data_ptr(), H * D * tp, D * tp, tp, out.data_ptr(), Tq * C, C,
-                      _ptr(attn_mask), ld, B, H, Tq, Tk, D, s["qm"], s["qs"], s["f"], s["am"],
+                      mp, ld, B, H, Tq, Tk, D, s["qm"], s["qs"], s["f"], s["am"],
                       s["as_"], self.rsqrt_offset, _ptr(table), decode, _stream())
             return out
         # Other head sizes: the three reference ops, each on the GPU.
@@ -369,8 +369,9 @@ class MultiHeadAttention_int(_ScalarCache, nn.Module):
         rm = torch.empty((B, H, Tq, 1), dtype=torch.int16, device=q.device)
         p = torch.empty((B, H, Tq, Tk), dtype=torch.uint8, device=q.device)
         rs = torch.empty((B, H, Tq, 1), dtype=torch.int32, device=q.device)
-        attn_mask = None if attn_mask is None else attn_mask.contiguous()
-        mp = _ptr(attn_mask)
+        if mask is not None:
+            mask = mask[q_offset:q_offset + Tq, :Tk].contiguous()
+        mp = _ptr(mask)
         _lib.call("iw_qk_requant_rowmax", qh.data_ptr(), kh.data_ptr(), mp, qk.data_ptr(),
                   rm.data_ptr(), B, H, Tq, Tk, D, s["qm"], s["qs"], mp is not None, _stream())
         _lib.call("iw_shift_exp", qk.data_ptr(), rm.data_ptr(), mp, p.data_ptr(), rs.data_ptr(), B,

@@ -146,6 +146,29 @@ def test_decoder_layers_read_the_mask_themselves(iw, small, n_tok):
     assert torch.equal(got, exp)
 
 
+@pytest.mark.parametrize("n_tok", [1, 6, 13])
+def test_attention_takes_masks_of_any_layout(iw, small, n_tok):
+    """A contiguous bool mask is read in place; slices, transposed views and byte masks are copied
+    first. All give what a mask of exactly these rows and keys gives, also behind cached keys."""
+    dims, P, model, ref = small
+    att = model.decoder.blocks[0].attn
+    r = gen.rng(n_tok)
+    x = T(gen.i8(r, (2, n_tok, 384), -127, 127))
+    keys = T(gen.i8(r, (2, n_tok + 4, 384), -127, 127))
+    full = r.random((32, 32)) < 0.4
+    full[:, 0] = False
+    m = T(full)
+    with torch.no_grad():
+        q, k, v = att.query(x), att.key(keys), att.value(keys)
+        for off in (0, 4):
+            kk, vv, tk = k[:, :n_tok + off], v[:, :n_tok + off], n_tok + off
+            exp = att.qkv_attention(q, kk, vv, m[:tk, :tk].contiguous())
+            plain = att.qkv_attention(q, kk, vv)
+            assert n_tok < 2 or not torch.equal(exp, plain)
+            for mask in (m, m[:tk], m[:, :tk], m.t().contiguous().t(), m.to(torch.uint8), m[:tk, :tk]):
+                assert torch.equal(att.qkv_attention(q, kk, vv, mask), exp)
+
+
 @pytest.mark.parametrize("batch,n_tok", [(2, 5), (9, 20)])
 def test_decoder_float_logits_by_either_way(iw, small, batch, n_tok):
     """The logits divided in one call (a one-element float32 alpha) and by classify and torch (alphas
